@@ -59,9 +59,10 @@ hipError_t deltanet_chunk_prefill_spin(const void* q, const void* k, const void*
 /* deltanet_chunk_prefill / _varlen (DK = DV = 128, chunk 64, dump_debug = 0)
  * with the scan instance chosen by the caller: slice_cols 16 runs one scan
  * work-group per 16 value columns of a (sequence, head), 32 the paired
- * instance with one per 32 columns, 0 the library's own choice (16 while the
- * 16-column groups fit on the device's CUs at once, 32 beyond).  Both give
- * bitwise the same o and final state.  cu_seqlens NULL: num_seqs sequences of
+ * instance with one per 32 columns, 128 the wide instance (the whole head: two
+ * work-groups of 64 columns), 0 the library's own choice (the narrowest whose
+ * groups fit on the device's CUs at once, else the wide one).  All give
+ * bitwise the same o and final state; the wide instance has no bounded waits.  cu_seqlens NULL: num_seqs sequences of
  * T tokens; otherwise a device array [num_seqs + 1] and T the total token
  * count.  spin_limit 0 keeps the library's bounded-wait limit, otherwise as in
  * deltanet_chunk_prefill_spin.  Other slice_cols: hipErrorInvalidValue. */

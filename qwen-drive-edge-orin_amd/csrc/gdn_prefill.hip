@@ -2401,6 +2401,267 @@ __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan2_kernel(ScanArgs a) 
     }
 }
 
+// ---------------------------------------------------------------------------
+// wide scan kernel: one work-group per (64 value columns, v-head, sequence),
+// for calls with more (sequence, v-head) pairs than the paired instance can
+// run at once.  The narrower instances keep the serial chain on a wave of its
+// own, so that one step is short, and leave most of a CU's matrix pipes idle;
+// once the groups run in rounds the CU time per chunk and column is what
+// counts.  Here each of four compute waves (one per SIMD) does everything for
+// 16 columns of its own (U, V_n, both state updates, O: 88 MFMAs a chunk) with
+// nothing handed from wave to wave, and four loader waves move the chunk's
+// whole operand set into LDS once for all 64 columns, a chunk ahead.
+//
+// LDS: two stages of 75 KB, one being read while the other fills; the waves
+// meet at one s_barrier per chunk.  Compute waves write no LDS and loaders
+// read none.  The arithmetic per 16 columns is the 16-column instance's,
+// operation for operation (o and the final state are bitwise the same).
+// ---------------------------------------------------------------------------
+constexpr int kWideCols = 64;
+constexpr int kWideSlices = kWideCols / kSliceCols;   // 4, one per compute wave
+constexpr int kWidesPerHead = kDV / kWideCols;        // 2
+constexpr int kWideHead = kDV;   // deltanet_chunk_prefill_cols: the wide instance, two groups a head
+constexpr int kWideLoaders = kScanWaves - kWideSlices;
+static_assert(kWideLoaders == 4, "the loaders split 16-fragment records in four");
+
+struct StageWide {
+    u32x4 KT[16][64];                   // K^T bf16 fragments (t * 2 + kb)
+    half8 W[16][64];                    // -W fragments (mt * 4 + kb)
+    half8 Q[16][64];                    // Q fragments (mt * 4 + kb)
+    half8 T[3][kTri][64];               // (T - I) hi, (T - I) lo, M
+    u32x4 V[kWideSlices][kChunk * 2];   // per slice: V rows of its 16 columns, 2 pieces per row
+    float gates[256];                   // gates record
+};
+
+struct ScanSmemWide {
+    StageWide st[2];
+    int seqsel;
+    int red[kScanWaves];
+};
+static_assert(sizeof(ScanSmemWide) <= 160 * 1024, "wide scan LDS");
+
+// s_barrier with this wave's LDS reads complete, and no memory operation
+// moved across it by the compiler
+__device__ __forceinline__ void wide_barrier() {
+    lds_wait_all();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Loader j (0..3): a quarter of each chunk's direct-to-LDS loads.  Chunk c + 1
+// goes into the stage that chunk c - 1 was read from, after the barrier that
+// ended chunk c - 1, and has landed before this wave enters the barrier that
+// ends chunk c.
+__device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanCtx& x, int j,
+                                int lane) {
+    auto issue = [&](int c) {
+        StageWide& st = sm.st[c & 1];
+        const size_t ck = (size_t)(x.chunk0 + c);
+        const size_t ch = ck * a.HV + x.hv;
+        // V rows of slice j: slot 64 i + lane -> row (64 i + lane) / 2, piece lane % 2
+        const int t0 = x.tok_base + c * kChunk, rows = min(kChunk, x.len - c * kChunk);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int s = 64 * i + lane, r = min(s >> 1, rows - 1);
+            lds_dma16(a.in.v + ((size_t)(t0 + r) * a.HV + x.hv) * kDV + kWideCols * x.sl +
+                          kSliceCols * j + 8 * (s & 1),
+                      &st.V[j][64 * i]);
+        }
+        if (j == kWideLoaders - 1)
+            lds_dma16(a.ws.gates + ch * (kGateBytes / 4) + 4 * lane, &st.gates[0]);
+        // fragments j, j + 4, .. of T - I hi, lo and M
+#pragma unroll
+        for (int f0 = 0; f0 < 3 * kTri; f0 += kWideLoaders) {
+            const int f = f0 + j;
+            if (f < 3 * kTri) {
+                const int reg = f / kTri, ff = f - reg * kTri;
+                const half8* src = reg == 0 ? a.ws.TI : reg == 1 ? a.ws.TIlo : a.ws.M;
+                lds_dma16(src + (ch * kTri + ff) * 64 + lane, &st.T[0][0][0] + f * 64);
+            }
+        }
+        const half8* wsrc = a.ws.W + (ch * 16 + 4 * j) * 64 + lane;
+        const size_t kq = ((ck * a.HK + x.hk) * 16 + 4 * j) * 64 + lane;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) lds_dma16(wsrc + f * 64, &st.W[4 * j + f][0]);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) lds_dma16(a.ws.KT + kq + f * 64, &st.KT[4 * j + f][0]);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) lds_dma16(a.ws.Q + kq + f * 64, &st.Q[4 * j + f][0]);
+    };
+    if (x.nch > 0) issue(0);
+    vm_wait_all();
+    wide_barrier();
+    for (int c = 0; c < x.nch; ++c) {
+        if (c + 1 < x.nch) issue(c + 1);
+        vm_wait_all();
+        wide_barrier();
+    }
+}
+
+// Compute wave j (0..3): columns 64 sl + 16 j .. + 15.
+template <int kRaw>
+__device__ void run_wide_compute(ScanSmemWide& sm, const ScanArgs& a, const ScanCtx& x, int j,
+                                 int lane) {
+    const int lg = lane >> 4, lm = lane & 15;
+    const int col0 = kWideCols * x.sl + kSliceCols * j;
+    auto dk_of = [&](int t, int i) { return 32 * (t >> 1) + 8 * lg + 4 * (t & 1) + i; };
+    const size_t sbase = ((size_t)x.seq * a.HV + x.hv) * kDK * kDV + col0 + lm;
+
+    f32x4 S[8], Sc[8];   // the state is S + Sc (run_chain)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        S[t] = zero4();
+        Sc[t] = zero4();
+    }
+    if (a.s0) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[t][i] = a.s0[sbase + (size_t)dk_of(t, i) * kDV];
+        }
+    }
+    half8 S16[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) S16[kb] = cat8(to_half4(S[2 * kb]), to_half4(S[2 * kb + 1]));
+
+    wide_barrier();   // chunk 0 is in
+    for (int c = 0; c < x.nch; ++c) {
+        const StageWide& st = sm.st[c & 1];
+        // U = beta V + (T - I)(beta V) (run_producer)
+        f32x4 Vn[4];
+        half8 xh[2], xl[2];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const f32x4 be = *reinterpret_cast<const f32x4*>(&st.gates[kGBeta + 16 * mt + 4 * lg]);
+            const uint16_t* vsrc = reinterpret_cast<const uint16_t*>(st.V[j]) +
+                                   (16 * mt + 4 * lg + (lm >> 2)) * kSliceCols + 4 * (lm & 3);
+            const s16x4 vt = lds_read_tr(vsrc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Vn[mt][i] = be[i] * v16_to_f32<kRaw>((uint16_t)vt[i]);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) split_hilo8(Vn[2 * kb], Vn[2 * kb + 1], xh[kb], xl[kb]);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                if (kb > mt / 2) break;
+                const half8 th = st.T[0][tri_base(mt) + kb][lane];
+                const half8 tl = st.T[1][tri_base(mt) + kb][lane];
+                Vn[mt] = mfma16(th, xh[kb], Vn[mt]);
+                Vn[mt] = mfma16(th, xl[kb], Vn[mt]);
+                Vn[mt] = mfma16(tl, xh[kb], Vn[mt]);
+            }
+        }
+        // V_n = U + (-W) S16, and O^T's state part S16^T Q^T beside it
+        f32x4 ov[4];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) ov[mt] = zero4();
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) {
+                Vn[mt] = mfma16(st.W[mt * 4 + kb][lane], S16[kb], Vn[mt]);
+                ov[mt] = mfma16(S16[kb], st.Q[mt * 4 + kb][lane], ov[mt]);
+            }
+        }
+        const float gam = __builtin_amdgcn_exp2f(st.gates[kGC63] * kLog2e);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            S[t] = S[t] * gam;
+            Sc[t] = Sc[t] * gam;
+        }
+        // d o V_n as a bf16 hi / lo pair
+        f32x4 dv[4];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            dv[mt] = *reinterpret_cast<const f32x4*>(&st.gates[kGDec + 16 * mt + 4 * lg]) * Vn[mt];
+            asm volatile("" : "+v"(dv[mt]));   // rounded here, as in run_chain
+        }
+        bf16x8 hi[2], lo[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            u32x4 hw, lw;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4& d = dv[2 * kb + (q >> 1)];
+                const int p = q & 1;
+                hw[q] = pack_bf16x2(d[2 * p], d[2 * p + 1]);
+                const float r0 = d[2 * p] - __uint_as_float(hw[q] << 16);
+                const float r1 = d[2 * p + 1] - __uint_as_float(hw[q] & 0xffff0000u);
+                lw[q] = pack_bf16x2(r0, r1);
+            }
+            hi[kb] = __builtin_bit_cast(bf16x8, hw);
+            lo[kb] = __builtin_bit_cast(bf16x8, lw);
+        }
+        // S <- e^{c63} S + K^T hi, Sc <- e^{c63} Sc + K^T lo
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const bf16x8 kt = __builtin_bit_cast(bf16x8, st.KT[t * 2 + kb][lane]);
+                S[t] = mfma16_bf16(kt, hi[kb], S[t]);
+                Sc[t] = mfma16_bf16(kt, lo[kb], Sc[t]);
+            }
+        }
+        // O^T = (S^T Q^T) diag(s e^c) + V_n^T M^T (run_output)
+        const half8 vh0 = cat8(to_half4(Vn[0]), to_half4(Vn[1]));
+        const half8 vh1 = cat8(to_half4(Vn[2]), to_half4(Vn[3]));
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            ov[mt] = ov[mt] * st.gates[kGSec + 16 * mt + lm];
+            ov[mt] = mfma16(vh0, st.T[2][tri_base(mt)][lane], ov[mt]);
+            if (mt >= 2) ov[mt] = mfma16(vh1, st.T[2][tri_base(mt) + 1][lane], ov[mt]);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) S16[kb] = cat8(to_half4(S[2 * kb]), to_half4(S[2 * kb + 1]));
+        const int rows = min(kChunk, x.len - c * kChunk);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const int r = 16 * mt + lm;
+            uint32_t b[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                b[e] = f32_to_bf16_bits(ov[mt][e]);
+                if constexpr (kRaw == 2) b[e] = f16_bits(__uint_as_float(b[e] << 16));
+            }
+            if (r < rows) {
+                uint2* dst = reinterpret_cast<uint2*>(
+                    a.o + ((size_t)(x.tok_base + c * kChunk + r) * a.HV + x.hv) * kDV + col0 + 4 * lg);
+                *dst = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+            }
+        }
+        wide_barrier();   // this stage may be refilled; the next one is in
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a.sf[sbase + (size_t)dk_of(t, i) * kDV] = S[t][i] + Sc[t][i];
+    }
+}
+
+template <int kRaw>
+__global__ __launch_bounds__(kScanThreads, 1) void gdn_scan_wide_kernel(ScanArgs a) {
+    __shared__ ScanSmemWide sm;
+    // kernel-argument lines requested together (as in gdn_scan_kernel)
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
+                 "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
+                 "s"(a.spin));
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // XCD-aware id: the two groups of one (sequence, head) share id % 8
+    const int id = blockIdx.x;
+    const int xcd = id & 7, qd = id >> 3;
+    ScanCtx x;
+    x.sl = qd % kWidesPerHead;
+    const int pidx = (qd / kWidesPerHead) * 8 + xcd;
+    if (pidx >= a.N * a.HV) return;
+    scan_context(a, pidx, &sm.seqsel, sm.red, x);
+    // wave w runs on SIMD w % 4: each compute wave shares its SIMD with a loader
+    if (wave < kWideSlices) run_wide_compute<kRaw>(sm, a, x, wave, lane);
+    else run_wide_loader(sm, a, x, wave - kWideSlices, lane);
+}
+
 // raw: 0 for prepared inputs, 1 / 2 for raw bf16 / fp16 q, k (normalised in
 // the prep; then v and o have that dtype too).
 // The gated-RMSNorm epilogue's inputs (bf16 z [token][HV][128], bf16 weight
@@ -2411,14 +2672,10 @@ struct NormIn {
     float eps;
 };
 
-// Scan work-groups of a call over N sequences of HV heads.
-inline long long scan_groups(int N, int HV) {
-    return (long long)((N * HV + 7) / 8) * 8 * kSlicesPerHead;
-}
-
-// ... and of the paired instance (32 columns per group).
-inline long long scan2_groups(int N, int HV) {
-    return (long long)((N * HV + 7) / 8) * 8 * kPairsPerHead;
+// Scan work-groups of a call over N sequences of HV heads, `cols` value
+// columns each.
+inline long long scan_groups(int N, int HV, int cols) {
+    return (long long)((N * HV + 7) / 8) * 8 * (kDV / cols);
 }
 
 // CUs of the current device (cached per device; 256 if the query fails).
@@ -2437,15 +2694,18 @@ int device_cus() {
     return n;
 }
 
-// Scan instance: 16-column groups while they fit on the CUs at once (one
-// group per CU), the paired 32-column groups once they would run in rounds
-// (then the halves' shared operands halve the rounds).  cols forces 16 or 32
-// (diagnostics); the debug dump and the norm epilogue exist in the 16-column
-// instance only.
-bool use_pair_scan(int cols, int N, int HV, int dump_debug, bool norm) {
-    if (cols == 32) return true;
-    if (cols == 16 || dump_debug || norm) return false;
-    return (long long)N * HV * kSlicesPerHead > device_cus();
+// Scan instance (value columns per work-group): 16-column groups while they
+// fit on the CUs at once (one group per CU), the paired 32-column groups once
+// they would run in rounds (then the halves' shared operands halve the
+// rounds), the wide 64-column groups once the paired ones would.  cols forces
+// one (diagnostics); the debug dump and the norm epilogue exist in the
+// 16-column instance only.
+int scan_cols(int cols, int N, int HV, int dump_debug, bool norm) {
+    if (cols) return cols;
+    if (dump_debug || norm) return kSliceCols;
+    const long long heads = (long long)N * HV, cus = device_cus();
+    if (heads * kSlicesPerHead <= cus) return kSliceCols;
+    return heads * kPairsPerHead <= cus ? kPairCols : kWideCols;
 }
 
 hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, float* sf,
@@ -2454,8 +2714,8 @@ hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, f
                           hipStream_t stream, int dump_debug, hipEvent_t* ev = nullptr,
                           int only = -1, unsigned spin = kDefaultSpin,
                           const NormIn* norm = nullptr, int cols = 0) {
-    const bool pair = use_pair_scan(cols, N, HV, dump_debug, norm != nullptr);
-    if (pair && (dump_debug || norm)) return hipErrorInvalidValue;
+    const int width = scan_cols(cols, N, HV, dump_debug, norm != nullptr);
+    if (width != kSliceCols && (dump_debug || norm)) return hipErrorInvalidValue;
     const WsLayout L(nch_bound * (size_t)HV);
     const size_t need = dump_debug ? L.total : L.live;
     if (workspace_bytes < need) return hipErrorInvalidValue;
@@ -2521,9 +2781,14 @@ hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, f
         sa.nw = norm->w;
         sa.eps = norm->eps;
     }
-    const unsigned grid = (unsigned)(pair ? scan2_groups(N, HV) : scan_groups(N, HV));
+    const unsigned grid = (unsigned)scan_groups(N, HV, width);
     hipError_t err;
-    if (pair) {
+    if (width == kWideCols) {
+        auto scan = raw == 1 ? gdn_scan_wide_kernel<1>
+                    : raw == 2 ? gdn_scan_wide_kernel<2> : gdn_scan_wide_kernel<0>;
+        hipLaunchKernelGGL(scan, dim3(grid), dim3(kScanThreads), 0, stream, sa);
+        err = hipGetLastError();
+    } else if (width == kPairCols) {
         auto scan = raw == 1 ? gdn_scan2_kernel<1> : raw == 2 ? gdn_scan2_kernel<2> : gdn_scan2_kernel<0>;
         hipLaunchKernelGGL(scan, dim3(grid), dim3(kScanThreads), 0, stream, sa);
         err = hipGetLastError();
@@ -2648,7 +2913,7 @@ extern "C" hipError_t deltanet_chunk_prefill_norm_fused(
     // The epilogue lives in the 16-column scan; where the plain prefill would
     // take the paired 32-column instance (more slice groups than CUs) the
     // two-kernel path runs instead.
-    if (use_pair_scan(0, B, HV, 0, false))
+    if (scan_cols(0, B, HV, 0, false) != kSliceCols)
         return prefill_then_norm(q, k, v, g, beta, z, norm_weight, eps, y, initial_state,
                                  final_state, B, T, HV, HQK, workspace, workspace_bytes, stream);
     const size_t nc = (size_t)B * ((T + kChunk - 1) / kChunk);
@@ -2690,8 +2955,10 @@ extern "C" hipError_t deltanet_chunk_prefill_cols(const void* q, const void* k, 
                                                   int HV, int HQK, void* workspace,
                                                   size_t workspace_bytes, hipStream_t stream,
                                                   int slice_cols, unsigned spin_limit) {
-    if (slice_cols != 0 && slice_cols != kSliceCols && slice_cols != kPairCols)
+    if (slice_cols != 0 && slice_cols != kSliceCols && slice_cols != kPairCols &&
+        slice_cols != kWideHead)
         return hipErrorInvalidValue;
+    if (slice_cols == kWideHead) slice_cols = kWideCols;
     if (!dims_ok(HV, HQK, kDK, kDV, kChunk) || num_seqs <= 0 || T < 0) return hipErrorInvalidValue;
     if (workspace == nullptr || final_state == nullptr) return hipErrorInvalidValue;
     if (T > 0 && (!q || !k || !v || !g || !beta || !o)) return hipErrorInvalidValue;
