@@ -2412,9 +2412,13 @@ __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan2_kernel(ScanArgs a) 
 // nothing handed from wave to wave, and four loader waves move the chunk's
 // whole operand set into LDS once for all 64 columns, a chunk ahead.
 //
-// LDS: two stages of 75 KB, one being read while the other fills; the waves
-// meet at one s_barrier per chunk.  Compute waves write no LDS and loaders
-// read none.  The arithmetic per 16 columns is the 16-column instance's,
+// LDS: a chunk's operands come in two parts, A (what V_n and S^T Q^T need) and
+// B (what the state update and V_n's part of O need), each with two stages.
+// Two barriers split a step: at M(c) every wave has read A(c), so A(c + 2) can
+// start to load, and at E(c) B(c), so B(c + 2) can; each part thus has one and
+// a half steps to arrive.  O leaves through LDS as whole 128-byte rows, stored
+// by the loaders (as 32-byte pieces from the compute waves it took 0.4 us a
+// step).  The arithmetic per 16 columns is the 16-column instance's,
 // operation for operation (o and the final state are bitwise the same).
 // ---------------------------------------------------------------------------
 constexpr int kWideCols = 64;
@@ -2422,25 +2426,36 @@ constexpr int kWideSlices = kWideCols / kSliceCols;   // 4, one per compute wave
 constexpr int kWidesPerHead = kDV / kWideCols;        // 2
 constexpr int kWideHead = kDV;   // deltanet_chunk_prefill_cols: the wide instance, two groups a head
 constexpr int kWideLoaders = kScanWaves - kWideSlices;
-static_assert(kWideLoaders == 4, "the loaders split 16-fragment records in four");
+static_assert(kWideLoaders == 4, "the loaders split records and rows in four");
 
-struct StageWide {
-    u32x4 KT[16][64];                   // K^T bf16 fragments (t * 2 + kb)
-    half8 W[16][64];                    // -W fragments (mt * 4 + kb)
-    half8 Q[16][64];                    // Q fragments (mt * 4 + kb)
-    half8 T[3][kTri][64];               // (T - I) hi, (T - I) lo, M
-    u32x4 V[kWideSlices][kChunk * 2];   // per slice: V rows of its 16 columns, 2 pieces per row
-    float gates[256];                   // gates record
+// V and O tiles: 64 rows (tokens) of 64 columns, 8 pieces of 16 bytes a row,
+// piece p of row r at slot 8 r + (p ^ r % 8): the 32 bytes that one wave
+// takes of 8 consecutive rows then fill the 64 banks once.
+__device__ __forceinline__ int wide_slot(int r, int p) { return 8 * r + (p ^ (r & 7)); }
+
+struct StageWideA {
+    half8 W[16][64];             // -W fragments (mt * 4 + kb)
+    half8 Q[16][64];             // Q fragments (mt * 4 + kb)
+    half8 T[2 * kTri][64];       // T - I: hi, then lo
+    u32x4 V[kChunk * 8];         // V rows (wide_slot)
+    float gates[256];            // gates record
+};
+
+struct StageWideB {
+    u32x4 KT[16][64];            // K^T bf16 fragments (t * 2 + kb)
+    half8 M[kTri][64];
 };
 
 struct ScanSmemWide {
-    StageWide st[2];
+    StageWideA a[2];
+    StageWideB b[2];
+    u32x4 O[kChunk * 8];         // O rows (wide_slot)
     int seqsel;
     int red[kScanWaves];
 };
 static_assert(sizeof(ScanSmemWide) <= 160 * 1024, "wide scan LDS");
 
-// s_barrier with this wave's LDS reads complete, and no memory operation
+// s_barrier with this wave's LDS operations complete, and no memory operation
 // moved across it by the compiler
 __device__ __forceinline__ void wide_barrier() {
     lds_wait_all();
@@ -2448,54 +2463,109 @@ __device__ __forceinline__ void wide_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// Loader j (0..3): a quarter of each chunk's direct-to-LDS loads.  Chunk c + 1
-// goes into the stage that chunk c - 1 was read from, after the barrier that
-// ended chunk c - 1, and has landed before this wave enters the barrier that
-// ends chunk c.
+// Loader j (0..3): a quarter of each chunk's direct-to-LDS loads, and rows
+// 16 j .. 16 j + 15 of O.  Loads complete in issue order, so "all but the
+// newest n" waits for the part that is needed next.  Every part is issued in
+// full (past the last chunk the last one again, into a stage that is no
+// longer read), so the counts hold; the stores of O are not counted on.
 __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanCtx& x, int j,
                                 int lane) {
-    auto issue = [&](int c) {
-        StageWide& st = sm.st[c & 1];
-        const size_t ck = (size_t)(x.chunk0 + c);
-        const size_t ch = ck * a.HV + x.hv;
-        // V rows of slice j: slot 64 i + lane -> row (64 i + lane) / 2, piece lane % 2
-        const int t0 = x.tok_base + c * kChunk, rows = min(kChunk, x.len - c * kChunk);
+    constexpr int kLoadsA = 4 + 4 + 3 + 2;   // W, Q, T, V (and the gates, loader 3)
+    constexpr int kLoadsB = 4 + 1;           // K^T, M (two fragments for loaders 0 and 1)
+    static_assert(3 * kWideLoaders == 2 * kTri, "T - I hi and lo in threes");
+    auto four = [&](const void* src, size_t rec, void* dst) {   // fragments 4 j .. 4 j + 3
+        const u32x4* sp = static_cast<const u32x4*>(src) + (rec * 16 + 4 * j) * 64 + lane;
+        u32x4* dp = static_cast<u32x4*>(dst) + 4 * j * 64;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int s = 64 * i + lane, r = min(s >> 1, rows - 1);
-            lds_dma16(a.in.v + ((size_t)(t0 + r) * a.HV + x.hv) * kDV + kWideCols * x.sl +
-                          kSliceCols * j + 8 * (s & 1),
-                      &st.V[j][64 * i]);
+        for (int f = 0; f < 4; ++f) lds_dma16(sp + f * 64, dp + f * 64);
+    };
+    // The two groups of a head (one L2) take its records in opposite orders:
+    // each then finds the half that the other brought in L2.
+    auto issue_a = [&](int cc) {
+        const int c = min(cc, x.nch - 1);
+        StageWideA& st = sm.a[cc & 1];
+        const size_t ck = (size_t)(x.chunk0 + c), ch = ck * a.HV + x.hv, kq = ck * a.HK + x.hk;
+        auto tri = [&] {   // fragments 3 j .. 3 j + 2 of hi and lo in a row
+            const half8* src = (j < 2 ? a.ws.TI : a.ws.TIlo) + (ch * kTri + 3 * (j & 1)) * 64 + lane;
+#pragma unroll
+            for (int f = 0; f < 3; ++f) lds_dma16(src + f * 64, &st.T[3 * j + f][0]);
+        };
+        if (x.sl == 0) {
+            tri();
+            four(a.ws.W, ch, st.W);
+            four(a.ws.Q, kq, st.Q);
+        } else {
+            four(a.ws.Q, kq, st.Q);
+            four(a.ws.W, ch, st.W);
+            tri();
         }
         if (j == kWideLoaders - 1)
             lds_dma16(a.ws.gates + ch * (kGateBytes / 4) + 4 * lane, &st.gates[0]);
-        // fragments j, j + 4, .. of T - I hi, lo and M
+        const int t0 = x.tok_base + c * kChunk, rows = min(kChunk, x.len - c * kChunk);
 #pragma unroll
-        for (int f0 = 0; f0 < 3 * kTri; f0 += kWideLoaders) {
-            const int f = f0 + j;
-            if (f < 3 * kTri) {
-                const int reg = f / kTri, ff = f - reg * kTri;
-                const half8* src = reg == 0 ? a.ws.TI : reg == 1 ? a.ws.TIlo : a.ws.M;
-                lds_dma16(src + (ch * kTri + ff) * 64 + lane, &st.T[0][0][0] + f * 64);
-            }
+        for (int i = 0; i < 2; ++i) {
+            const int r = 16 * j + 8 * i + (lane >> 3), p = (lane ^ r) & 7;   // slot 8 r + lane % 8
+            lds_dma16(a.in.v + ((size_t)(t0 + min(r, rows - 1)) * a.HV + x.hv) * kDV +
+                          kWideCols * x.sl + 8 * p,
+                      &st.V[(16 * j + 8 * i) * 8]);
         }
-        const half8* wsrc = a.ws.W + (ch * 16 + 4 * j) * 64 + lane;
-        const size_t kq = ((ck * a.HK + x.hk) * 16 + 4 * j) * 64 + lane;
-#pragma unroll
-        for (int f = 0; f < 4; ++f) lds_dma16(wsrc + f * 64, &st.W[4 * j + f][0]);
-#pragma unroll
-        for (int f = 0; f < 4; ++f) lds_dma16(a.ws.KT + kq + f * 64, &st.KT[4 * j + f][0]);
-#pragma unroll
-        for (int f = 0; f < 4; ++f) lds_dma16(a.ws.Q + kq + f * 64, &st.Q[4 * j + f][0]);
     };
-    if (x.nch > 0) issue(0);
-    vm_wait_all();
+    auto issue_b = [&](int cc) {
+        const int c = min(cc, x.nch - 1);
+        StageWideB& st = sm.b[cc & 1];
+        const size_t ck = (size_t)(x.chunk0 + c), ch = ck * a.HV + x.hv;
+        if (x.sl == 0) four(a.ws.KT, ck * a.HK + x.hk, st.KT);
+        const half8* src = a.ws.M + (ch * kTri + j) * 64 + lane;
+        lds_dma16(src, &st.M[j][0]);
+        if (j < kTri - kWideLoaders) lds_dma16(src + kWideLoaders * 64, &st.M[j + kWideLoaders][0]);
+        if (x.sl != 0) four(a.ws.KT, ck * a.HK + x.hk, st.KT);
+    };
+    // O of chunk c, rows 16 j .. + 15.  The reads and their wait are one asm
+    // block: the compiler would place a wait for every direct-to-LDS load in
+    // front of an LDS read of its own.
+    auto store_o = [&](int c) {
+        const int rows = min(kChunk, x.len - c * kChunk);
+        u32x4 v0, v1;
+        const uint32_t addr =
+            (uint32_t)(size_t)(__attribute__((address_space(3))) u32x4*)&sm.O[16 * j * 8 + lane];
+        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:1024\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(v0), "=&v"(v1)
+                     : "v"(addr)
+                     : "memory");
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = 16 * j + 8 * i + (lane >> 3), p = (lane ^ r) & 7;
+            if (r < rows)
+                *reinterpret_cast<u32x4*>(
+                    a.o + ((size_t)(x.tok_base + c * kChunk + r) * a.HV + x.hv) * kDV +
+                    kWideCols * x.sl + 8 * p) = i ? v1 : v0;
+        }
+    };
+    if (x.nch <= 0) return;
+    auto fence = [] { asm volatile("" ::: "memory"); };   // keeps the parts' issue order
+    issue_a(0);
+    fence();
+    issue_b(0);
+    fence();
+    issue_a(1);
+    fence();
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoadsA));   // A(0), B(0)
     wide_barrier();
     for (int c = 0; c < x.nch; ++c) {
-        if (c + 1 < x.nch) issue(c + 1);
-        vm_wait_all();
-        wide_barrier();
+        if (c > 0) store_o(c - 1);
+        fence();
+        issue_b(c + 1);
+        fence();
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoadsA + kLoadsB));   // up to B(c)
+        wide_barrier();                                             // M(c)
+        issue_a(c + 2);
+        fence();
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(kLoadsB + kLoadsA));   // up to A(c + 1)
+        wide_barrier();                                             // E(c)
     }
+    store_o(x.nch - 1);
+    vm_wait_all();   // no load may land in LDS after the group ends
 }
 
 // Compute wave j (0..3): columns 64 sl + 16 j .. + 15.
@@ -2503,9 +2573,9 @@ template <int kRaw>
 __device__ void run_wide_compute(ScanSmemWide& sm, const ScanArgs& a, const ScanCtx& x, int j,
                                  int lane) {
     const int lg = lane >> 4, lm = lane & 15;
-    const int col0 = kWideCols * x.sl + kSliceCols * j;
     auto dk_of = [&](int t, int i) { return 32 * (t >> 1) + 8 * lg + 4 * (t & 1) + i; };
-    const size_t sbase = ((size_t)x.seq * a.HV + x.hv) * kDK * kDV + col0 + lm;
+    const size_t sbase =
+        ((size_t)x.seq * a.HV + x.hv) * kDK * kDV + kWideCols * x.sl + kSliceCols * j + lm;
 
     f32x4 S[8], Sc[8];   // the state is S + Sc (run_chain)
 #pragma unroll
@@ -2524,63 +2594,130 @@ __device__ void run_wide_compute(ScanSmemWide& sm, const ScanArgs& a, const Scan
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) S16[kb] = cat8(to_half4(S[2 * kb]), to_half4(S[2 * kb + 1]));
 
-    wide_barrier();   // chunk 0 is in
+    if (x.nch > 0) wide_barrier();   // A(0) and B(0) are in
     for (int c = 0; c < x.nch; ++c) {
-        const StageWide& st = sm.st[c & 1];
-        // U = beta V + (T - I)(beta V) (run_producer)
-        f32x4 Vn[4];
-        half8 xh[2], xl[2];
+        const StageWideA& st = sm.a[c & 1];
+        const StageWideB& sb = sm.b[c & 1];
+        // A wave issues in order: operands are read a group of products
+        // ahead, and each group of products has the VALU work that later
+        // groups need placed between its members.
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        // (1) O^T's state part S16^T Q^T, which needs only the state, beside
+        // X = beta V and its hi / lo split (run_producer)
+        f32x4 Vn[4], ov[4], be[4];
+        s16x4 vt[4];
+        half8 qf[16];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            const f32x4 be = *reinterpret_cast<const f32x4*>(&st.gates[kGBeta + 16 * mt + 4 * lg]);
-            const uint16_t* vsrc = reinterpret_cast<const uint16_t*>(st.V[j]) +
-                                   (16 * mt + 4 * lg + (lm >> 2)) * kSliceCols + 4 * (lm & 3);
-            const s16x4 vt = lds_read_tr(vsrc);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) Vn[mt][i] = be[i] * v16_to_f32<kRaw>((uint16_t)vt[i]);
+            be[mt] = *reinterpret_cast<const f32x4*>(&st.gates[kGBeta + 16 * mt + 4 * lg]);
+            const int r = 16 * mt + 4 * lg + (lm >> 2);
+            vt[mt] = lds_read_tr(reinterpret_cast<const uint16_t*>(&st.V[wide_slot(r, 2 * j + ((lm >> 1) & 1))]) +
+                                 4 * (lm & 1));
         }
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) split_hilo8(Vn[2 * kb], Vn[2 * kb + 1], xh[kb], xl[kb]);
+        for (int f = 0; f < 4; ++f) {
+            qf[4 * f] = st.Q[4 * f][lane];
+            qf[4 * f + 1] = st.Q[4 * f + 1][lane];
+        }
+        fence();
+        half8 xh[2], xl[2], tf[2][kTri];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
+            ov[mt] = mfma16(S16[0], qf[4 * mt], zero4());
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                if (kb > mt / 2) break;
-                const half8 th = st.T[0][tri_base(mt) + kb][lane];
-                const half8 tl = st.T[1][tri_base(mt) + kb][lane];
-                Vn[mt] = mfma16(th, xh[kb], Vn[mt]);
-                Vn[mt] = mfma16(th, xl[kb], Vn[mt]);
-                Vn[mt] = mfma16(tl, xh[kb], Vn[mt]);
-            }
+            for (int i = 0; i < 4; ++i) Vn[mt][i] = be[mt][i] * v16_to_f32<kRaw>((uint16_t)vt[mt][i]);
+            qf[4 * mt + 2] = st.Q[4 * mt + 2][lane];
+            qf[4 * mt + 3] = st.Q[4 * mt + 3][lane];
+            fence();
         }
-        // V_n = U + (-W) S16, and O^T's state part S16^T Q^T beside it
-        f32x4 ov[4];
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) ov[mt] = zero4();
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
-                Vn[mt] = mfma16(st.W[mt * 4 + kb][lane], S16[kb], Vn[mt]);
-                ov[mt] = mfma16(S16[kb], st.Q[mt * 4 + kb][lane], ov[mt]);
-            }
-        }
-        const float gam = __builtin_amdgcn_exp2f(st.gates[kGC63] * kLog2e);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            S[t] = S[t] * gam;
-            Sc[t] = Sc[t] * gam;
-        }
-        // d o V_n as a bf16 hi / lo pair
-        f32x4 dv[4];
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            dv[mt] = *reinterpret_cast<const f32x4*>(&st.gates[kGDec + 16 * mt + 4 * lg]) * Vn[mt];
-            asm volatile("" : "+v"(dv[mt]));   // rounded here, as in run_chain
-        }
-        bf16x8 hi[2], lo[2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
+            // hi, then the residual, of one packed operand (split_hilo8)
+            half8 h = cat8(to_half4(Vn[2 * kb]), to_half4(Vn[2 * kb + 1]));
+            asm("" : "+v"(h));
+            f32x4 ra, rb;
+            ov[0] = mfma16(S16[kb + 1], qf[kb + 1], ov[0]);
+            tf[0][3 * kb] = st.T[3 * kb][lane];
+            fence();
+            ov[1] = mfma16(S16[kb + 1], qf[4 + kb + 1], ov[1]);
+            tf[0][3 * kb + 1] = st.T[3 * kb + 1][lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ra[i] = Vn[2 * kb][i] - (float)h[i];
+            fence();
+            ov[2] = mfma16(S16[kb + 1], qf[8 + kb + 1], ov[2]);
+            tf[0][3 * kb + 2] = st.T[3 * kb + 2][lane];
+            tf[1][3 * kb] = st.T[kTri + 3 * kb][lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rb[i] = Vn[2 * kb + 1][i] - (float)h[4 + i];
+            fence();
+            ov[3] = mfma16(S16[kb + 1], qf[12 + kb + 1], ov[3]);
+            tf[1][3 * kb + 1] = st.T[kTri + 3 * kb + 1][lane];
+            tf[1][3 * kb + 2] = st.T[kTri + 3 * kb + 2][lane];
+            xh[kb] = h;
+            xl[kb] = cat8(to_half4(ra), to_half4(rb));
+            fence();
+        }
+        // (2) U = X + (T - I) X, then V_n = U + (-W) S16, four row tiles at a
+        // time; the state's decay beside them
+        const float c63 = st.gates[kGC63];
+        half8 wf[16];
+        f32x4 dec[4];
+        float es[4];
+        auto read_w = [&](int f) { wf[f] = st.W[f][lane]; };
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {   // token k-block 0, hi hi
+            Vn[mt] = mfma16(tf[0][tri_base(mt)], xh[0], Vn[mt]);
+            ov[mt] = mfma16(S16[3], qf[4 * mt + 3], ov[mt]);
+            read_w(4 * mt);
+            read_w(4 * mt + 3);
+            fence();
+        }
+        const float gam = __builtin_amdgcn_exp2f(c63 * kLog2e);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {   // hi lo
+            Vn[mt] = mfma16(tf[0][tri_base(mt)], xl[0], Vn[mt]);
+            read_w(4 * mt + 1);
+            dec[mt] = *reinterpret_cast<const f32x4*>(&st.gates[kGDec + 16 * mt + 4 * lg]);
+            S[mt] = S[mt] * gam;
+            fence();
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {   // lo hi
+            Vn[mt] = mfma16(tf[1][tri_base(mt)], xh[0], Vn[mt]);
+            read_w(4 * mt + 2);
+            es[mt] = st.gates[kGSec + 16 * mt + lm];
+            S[4 + mt] = S[4 + mt] * gam;
+            fence();
+        }
+        // row tiles 2 and 3 have a second token k-block; 0 and 1 go on to -W
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+#pragma unroll
+            for (int mt = 2; mt < 4; ++mt) {
+                Vn[mt] = mfma16(tf[p / 2][tri_base(mt) + 1], p == 1 ? xl[1] : xh[1], Vn[mt]);
+                Vn[mt - 2] = mfma16(wf[4 * (mt - 2) + p], S16[p], Vn[mt - 2]);
+                Sc[2 * p + mt - 2] = Sc[2 * p + mt - 2] * gam;
+                fence();
+            }
+        }
+        wide_barrier();   // M(c): A(c) is in registers; B(c) is in
+        bf16x8 kt[16];
+        auto read_kt = [&](int t, int kb) { kt[t * 2 + kb] = __builtin_bit_cast(bf16x8, sb.KT[t * 2 + kb][lane]); };
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+            Vn[mt] = mfma16(wf[4 * mt + 3], S16[3], Vn[mt]);
+            Vn[2] = mfma16(wf[8 + mt], S16[mt], Vn[2]);
+            Vn[3] = mfma16(wf[12 + mt], S16[mt], Vn[3]);
+            Sc[6 + mt] = Sc[6 + mt] * gam;
+            read_kt(2 * mt, 0);
+            read_kt(2 * mt + 1, 0);
+            fence();
+        }
+        // (3) d o V_n as a bf16 hi / lo pair and V_n as fp16, token k-block 0
+        // while row tiles 2 and 3 finish
+        f32x4 dv[4];
+        bf16x8 hi[2], lo[2];
+        auto split_dv = [&](int kb) {
             u32x4 hw, lw;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -2593,45 +2730,67 @@ __device__ void run_wide_compute(ScanSmemWide& sm, const ScanArgs& a, const Scan
             }
             hi[kb] = __builtin_bit_cast(bf16x8, hw);
             lo[kb] = __builtin_bit_cast(bf16x8, lw);
-        }
-        // S <- e^{c63} S + K^T hi, Sc <- e^{c63} Sc + K^T lo
+        };
+        auto scale_dv = [&](int mt) {
+            dv[mt] = dec[mt] * Vn[mt];
+            asm("" : "+v"(dv[mt]));   // rounded here, as in run_chain
+        };
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const bf16x8 kt = __builtin_bit_cast(bf16x8, st.KT[t * 2 + kb][lane]);
-                S[t] = mfma16_bf16(kt, hi[kb], S[t]);
-                Sc[t] = mfma16_bf16(kt, lo[kb], Sc[t]);
-            }
+        for (int p = 2; p < 4; ++p) {
+            Vn[2] = mfma16(wf[8 + p], S16[p], Vn[2]);
+            Vn[3] = mfma16(wf[12 + p], S16[p], Vn[3]);
+            scale_dv(p - 2);
+            read_kt(2 * p, 0);
+            read_kt(2 * p + 1, 0);
+            fence();
         }
-        // O^T = (S^T Q^T) diag(s e^c) + V_n^T M^T (run_output)
+        split_dv(0);
         const half8 vh0 = cat8(to_half4(Vn[0]), to_half4(Vn[1]));
-        const half8 vh1 = cat8(to_half4(Vn[2]), to_half4(Vn[3]));
+        half8 mf[kTri];
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            ov[mt] = ov[mt] * st.gates[kGSec + 16 * mt + lm];
-            ov[mt] = mfma16(vh0, st.T[2][tri_base(mt)][lane], ov[mt]);
-            if (mt >= 2) ov[mt] = mfma16(vh1, st.T[2][tri_base(mt) + 1][lane], ov[mt]);
+        for (int f = 0; f < kTri; ++f) mf[f] = sb.M[f][lane];
+        fence();
+        // (4) S <- e^{c63} S + K^T hi, Sc <- e^{c63} Sc + K^T lo, and
+        // O^T += V_n^T M^T (run_output) between them
+        half8 vh1;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            S[t] = mfma16_bf16(kt[t * 2], hi[0], S[t]);
+            if (t < 2) scale_dv(2 + t);
+            if (t == 2) split_dv(1);
+            if (t == 3) vh1 = cat8(to_half4(Vn[2]), to_half4(Vn[3]));
+            Sc[t] = mfma16_bf16(kt[t * 2], lo[0], Sc[t]);
+            read_kt(t, 1);
+            if (t >= 4) ov[t - 4] = ov[t - 4] * es[t - 4];
+            fence();
         }
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) S16[kb] = cat8(to_half4(S[2 * kb]), to_half4(S[2 * kb + 1]));
-        const int rows = min(kChunk, x.len - c * kChunk);
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            const int r = 16 * mt + lm;
-            uint32_t b[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                b[e] = f32_to_bf16_bits(ov[mt][e]);
-                if constexpr (kRaw == 2) b[e] = f16_bits(__uint_as_float(b[e] << 16));
-            }
-            if (r < rows) {
-                uint2* dst = reinterpret_cast<uint2*>(
-                    a.o + ((size_t)(x.tok_base + c * kChunk + r) * a.HV + x.hv) * kDV + col0 + 4 * lg);
-                *dst = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
-            }
+        for (int t = 0; t < 8; ++t) {
+            S[t] = mfma16_bf16(kt[t * 2 + 1], hi[1], S[t]);
+            if (t < 4) ov[t] = mfma16(vh0, mf[tri_base(t)], ov[t]);
+            else if (t < 6) ov[t - 2] = mfma16(vh1, mf[tri_base(t - 2) + 1], ov[t - 2]);
+            if (t >= 2 && (t & 1) == 0) S16[(t >> 1) - 1] = cat8(to_half4(S[t - 2]), to_half4(S[t - 1]));
+            fence();
         }
-        wide_barrier();   // this stage may be refilled; the next one is in
+        // lane (lg, lm) of tile mt holds columns 4 lg .. + 3 of token 16 mt + lm
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            Sc[t] = mfma16_bf16(kt[t * 2 + 1], lo[1], Sc[t]);
+            if (t & 1) {
+                const int mt = t >> 1, r = 16 * mt + lm;
+                uint32_t b[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    b[e] = f32_to_bf16_bits(ov[mt][e]);
+                    if constexpr (kRaw == 2) b[e] = f16_bits(__uint_as_float(b[e] << 16));
+                }
+                reinterpret_cast<uint2*>(&sm.O[wide_slot(r, 2 * j + (lg >> 1))])[lg & 1] =
+                    make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+            }
+            fence();
+        }
+        S16[3] = cat8(to_half4(S[6]), to_half4(S[7]));
+        wide_barrier();   // E(c): O(c) is written, B(c) is in registers; A(c + 1) is in
     }
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
