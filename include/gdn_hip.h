@@ -217,6 +217,32 @@ hipError_t deltanet_recurrent_step_l2norm(const void* q, const void* k, const vo
                                           float* state, int B, int T, int HV, int HQK, int DK,
                                           int DV, hipStream_t stream);
 
+/* deltanet_recurrent_step (qk_l2norm != 0: _l2norm) for q, k, v rows that lie
+ * apart, and for a state that goes to another buffer: heads lie next to each
+ * other (128 elements), batches and tokens q_batch, q_token, .. elements
+ * apart (below 2^31); v 8-byte aligned, its strides multiples of 4.  state_in NULL: zeros;
+ * state_in may be state_out.  Head dims 128.  T = 0 needs state_in =
+ * state_out (nothing is done). */
+hipError_t deltanet_recurrent_step_strided(const void* q, const void* k, const void* v,
+                                           const float* g, const float* beta, void* o,
+                                           const float* state_in, float* state_out, int B, int T,
+                                           int HV, int HQK, int64_t q_batch, int64_t q_token,
+                                           int64_t k_batch, int64_t k_token, int64_t v_batch,
+                                           int64_t v_token, int qk_l2norm, hipStream_t stream);
+
+/* deltanet_chunk_prefill / _varlen (cu_seqlens NULL or not), qk_l2norm != 0:
+ * with q and k normalised in the kernels, for q, k, v rows that lie apart:
+ * heads next to each other, tokens (over the whole batch: sequence b's token
+ * t is token b T + t) q_token, k_token, v_token elements apart, multiples of
+ * 8 and below 2^31; q, k, v 16-byte aligned.  o is packed.  No debug views. */
+hipError_t deltanet_chunk_prefill_strided(const void* q, int64_t q_token, const void* k,
+                                          int64_t k_token, const void* v, int64_t v_token,
+                                          const float* g, const float* beta, void* o,
+                                          const float* initial_state, float* final_state,
+                                          const int32_t* cu_seqlens, int num_seqs, int B, int T,
+                                          int HV, int HQK, int qk_l2norm, void* workspace,
+                                          size_t workspace_bytes, hipStream_t stream);
+
 /* Gated RMSNorm y = rmsnorm(x) * w * silu(z) over rows of dv elements.
  * Replaces kernel::gatedRmsNormForward (export/patches/orin_text_engine/files/
  * cpp/kernels/gatedRmsNorm/gatedRmsNormKernel.h:17-18), which was fp16-only.

@@ -159,6 +159,9 @@ struct PrepIn {
     const float* A_log;
     const uint16_t* dt_bias;
     const float* s0;   // the scan's initial state (the prep only touches it)
+    // elements from a token's q, k or v row of head 0 to the next token's
+    // (over the whole batch; heads lie next to each other), negative: packed
+    int qts = -1, kts = -1, vts = -1;
 };
 
 // ---------------------------------------------------------------------------
@@ -480,7 +483,7 @@ __global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(
     // scalar cache would otherwise fetch in three dependent round trips (each
     // use waits before the branch that leads to the next): fields at most 32
     // bytes apart, all requested together, cost one.
-    asm volatile("" ::"s"(in.q), "s"(in.A_log), "s"(cu), "s"(nch_bound), "s"(ws.TIlo),
+    asm volatile("" ::"s"(in.q), "s"(in.A_log), "s"(in.kts), "s"(cu), "s"(nch_bound), "s"(ws.TIlo),
                  "s"(ws.gates), "s"(ws.ncnt), "s"(ws.dbgT), "s"(ws.dbgM), "s"(ws.dbgS));
     const uint16_t* __restrict__ q = in.q;
     const uint16_t* __restrict__ k = in.k;
@@ -538,18 +541,18 @@ __global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(
     // K: thread tid holds piece tid % 16 of rows tid / 16 + 16 ii
     u32x4 raw[4];
     {
-        const uint16_t* base = k + ((size_t)tok0 * HK + hk) * kDK + 8 * (tid & 15);
+        const uint16_t* base = k + (size_t)tok0 * in.kts + hk * kDK + 8 * (tid & 15);
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii) {
             const int r = min((tid >> 4) + 16 * ii, rows - 1);
-            raw[ii] = *reinterpret_cast<const u32x4*>(base + (size_t)r * HK * kDK);
+            raw[ii] = *reinterpret_cast<const u32x4*>(base + (size_t)r * in.kts);
         }
     }
     // Q: wave w, lane (lg, lm) holds row 16 w + lm, dk 32 kb + 8 lg .. + 7
     u32x4 qr[4];
     {
         const uint16_t* qs =
-            q + ((size_t)(tok0 + min(wave * 16 + lm, rows - 1)) * HK + hk) * kDK + 8 * lg;
+            q + (size_t)(tok0 + min(wave * 16 + lm, rows - 1)) * in.qts + hk * kDK + 8 * lg;
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) qr[kb] = *reinterpret_cast<const u32x4*>(qs + kb * 32);
     }
@@ -1077,7 +1080,7 @@ __device__ void run_loader(ScanSmem& sm, const ScanArgs& a, const Waiter& w, con
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int s = 64 * i + lane, r = min(s >> 1, rows - 1);
-            lds_dma16(a.in.v + ((size_t)(t0 + r) * a.HV + x.hv) * kDV + kSliceCols * x.sl + 8 * (s & 1),
+            lds_dma16(a.in.v + (size_t)(t0 + r) * a.in.vts + x.hv * kDV + kSliceCols * x.sl + 8 * (s & 1),
                       &st.V[64 * i]);
         }
         lds_dma16(a.ws.gates + ch_of(c) * (kGateBytes / 4) + 4 * lane, &st.gates[0]);
@@ -1774,7 +1777,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan_kernel(ScanArgs a) {
     // The kernel arguments (288 bytes) span five 64-byte lines, which the
     // scalar cache would otherwise fetch in three dependent round trips:
     // fields at most 32 bytes apart, all requested together, cost one.
-    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.in.vts), "s"(a.ws.M), "s"(a.ws.KT),
                  "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
                  "s"(a.spin));
     const int tid = threadIdx.x;
@@ -1941,7 +1944,7 @@ __device__ void run_loader2(ScanSmem2& sm, const ScanArgs& a, const Waiter& w, c
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int s = 64 * i + lane, r = min(s >> 1, rows - 1);
-                lds_dma16(a.in.v + ((size_t)(t0 + r) * a.HV + x.hv) * kDV + kPairCols * x.sl +
+                lds_dma16(a.in.v + (size_t)(t0 + r) * a.in.vts + x.hv * kDV + kPairCols * x.sl +
                               kSliceCols * h + 8 * (s & 1),
                           &sp.V[h][64 * i]);
             }
@@ -2359,7 +2362,7 @@ template <int kRaw>
 __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan2_kernel(ScanArgs a) {
     __shared__ ScanSmem2 sm;
     // kernel-argument lines requested together (as in gdn_scan_kernel)
-    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.in.vts), "s"(a.ws.M), "s"(a.ws.KT),
                  "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
                  "s"(a.spin));
     const int tid = threadIdx.x;
@@ -2508,7 +2511,7 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int r = 16 * j + 8 * i + (lane >> 3), p = (lane ^ r) & 7;   // slot 8 r + lane % 8
-            lds_dma16(a.in.v + ((size_t)(t0 + min(r, rows - 1)) * a.HV + x.hv) * kDV +
+            lds_dma16(a.in.v + (size_t)(t0 + min(r, rows - 1)) * a.in.vts + x.hv * kDV +
                           kWideCols * x.sl + 8 * p,
                       &st.V[(16 * j + 8 * i) * 8]);
         }
@@ -2806,7 +2809,7 @@ template <int kRaw>
 __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan_wide_kernel(ScanArgs a) {
     __shared__ ScanSmemWide sm;
     // kernel-argument lines requested together (as in gdn_scan_kernel)
-    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.in.vts), "s"(a.ws.M), "s"(a.ws.KT),
                  "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
                  "s"(a.spin));
     const int tid = threadIdx.x;
@@ -2870,7 +2873,7 @@ int scan_cols(int cols, int N, int HV, int dump_debug, bool norm) {
     return heads * kPairsPerHead <= cus ? kPairCols : kWideCols;
 }
 
-hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, float* sf,
+hipError_t launch_prefill(PrepIn in, int raw, void* o, const float* s0, float* sf,
                           const int32_t* cu, int N, int T, int total_tokens, int HV, int HK,
                           size_t nch_bound, void* workspace, size_t workspace_bytes,
                           hipStream_t stream, int dump_debug, hipEvent_t* ev = nullptr,
@@ -2878,6 +2881,9 @@ hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, f
                           const NormIn* norm = nullptr, int cols = 0) {
     const int width = scan_cols(cols, N, HV, dump_debug, norm != nullptr);
     if (width != kSliceCols && (dump_debug || norm)) return hipErrorInvalidValue;
+    if (in.qts < 0) in.qts = HK * kDK;
+    if (in.kts < 0) in.kts = HK * kDK;
+    if (in.vts < 0) in.vts = HV * kDV;
     const WsLayout L(nch_bound * (size_t)HV);
     const size_t need = dump_debug ? L.total : L.live;
     if (workspace_bytes < need) return hipErrorInvalidValue;
@@ -3341,6 +3347,37 @@ extern "C" hipError_t deltanet_chunk_prefill_fused(const void* q, const void* k,
     const size_t nc = (size_t)B * ((T + kChunk - 1) / kChunk);
     return launch_prefill(in, io_dtype == GDN_DTYPE_FP16 ? 2 : 1, o, state, state, nullptr, B, T,
                           B * T, HV, HQK, nc, workspace, workspace_bytes, stream, 0);
+}
+
+// cu_seqlens NULL: B sequences of T tokens; else packed, num_seqs sequences of
+// T tokens in total (B must be 1).
+extern "C" hipError_t deltanet_chunk_prefill_strided(
+    const void* q, int64_t q_token, const void* k, int64_t k_token, const void* v,
+    int64_t v_token, const float* g, const float* beta, void* o, const float* initial_state,
+    float* final_state, const int32_t* cu_seqlens, int num_seqs, int B, int T, int HV, int HQK,
+    int qk_l2norm, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    if (!dims_ok(HV, HQK, kDK, kDV, kChunk) || B <= 0 || T < 0) return hipErrorInvalidValue;
+    if (cu_seqlens && (B != 1 || num_seqs <= 0)) return hipErrorInvalidValue;
+    if (workspace == nullptr || final_state == nullptr) return hipErrorInvalidValue;
+    if (T > 0 && (!q || !k || !v || !g || !beta || !o)) return hipErrorInvalidValue;
+    // rows are read 16 bytes at a time
+    for (int64_t t : {q_token, k_token, v_token})
+        if (t < 0 || t > 0x7fffffff || t % 8) return hipErrorInvalidValue;
+    for (const void* p : {q, k, v})
+        if (reinterpret_cast<uintptr_t>(p) % 16) return hipErrorInvalidValue;
+    PrepIn in = plain_in(q, k, v, g, beta);
+    in.qts = (int)q_token;
+    in.kts = (int)k_token;
+    in.vts = (int)v_token;
+    const int raw = qk_l2norm ? 1 : 0;
+    if (cu_seqlens) {
+        const size_t nc = ((size_t)T + (size_t)(kChunk - 1) * num_seqs) / kChunk;
+        return launch_prefill(in, raw, o, initial_state, final_state, cu_seqlens, num_seqs, 0, T,
+                              HV, HQK, nc, workspace, workspace_bytes, stream, 0);
+    }
+    const size_t nc = (size_t)B * ((T + kChunk - 1) / kChunk);
+    return launch_prefill(in, raw, o, initial_state, final_state, nullptr, B, T, B * T, HV, HQK,
+                          nc, workspace, workspace_bytes, stream, 0);
 }
 
 // As deltanet_chunk_prefill / _varlen, with q and k rows L2-normalised in the

@@ -38,6 +38,26 @@ void check_hip(hipError_t err, const char* what) {
     TORCH_CHECK(err == hipSuccess, what, " failed: ", hipGetErrorString(err));
 }
 
+// x [B, T, H, 128] as the kernels read it in place: a head's elements and the
+// heads next to each other, 16-byte aligned rows; anything else is copied.
+at::Tensor head_rows(const at::Tensor& x) {
+    const int64_t H = x.size(2), D = x.size(3);
+    const bool ok = x.stride(3) == 1 && (H <= 1 || x.stride(2) == D) &&
+                    (x.size(0) <= 1 || (x.stride(0) % 8 == 0 && x.stride(0) <= 0x7fffffff)) &&
+                    (x.size(1) <= 1 || (x.stride(1) % 8 == 0 && x.stride(1) <= 0x7fffffff));
+    at::Tensor r = ok ? x : x.contiguous();
+    return reinterpret_cast<uintptr_t>(r.data_ptr()) % 16 == 0 ? r : r.clone(at::MemoryFormat::Contiguous);
+}
+
+// The same with the tokens of the whole batch one stride apart, and that stride
+at::Tensor token_rows(const at::Tensor& x, int64_t& token) {
+    at::Tensor r = head_rows(x);
+    const int64_t B = r.size(0), T = r.size(1);
+    if (B > 1 && T > 1 && r.stride(0) != T * r.stride(1)) r = r.contiguous();
+    token = T > 1 ? r.stride(1) : B > 1 ? r.stride(0) : r.size(2) * r.size(3);
+    return r;
+}
+
 std::vector<at::Tensor> chunk_prefill_impl(const at::Tensor& q, const at::Tensor& k,
                                            const at::Tensor& v, const at::Tensor& g,
                                            const at::Tensor& beta,
@@ -56,9 +76,12 @@ std::vector<at::Tensor> chunk_prefill_impl(const at::Tensor& q, const at::Tensor
                 "bad ranks");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
 
-    auto qc = q.contiguous();
-    auto kc = k.contiguous();
-    auto vc = v.contiguous();
+    // the debug and test entries take packed rows, the others strided ones
+    const bool packed = debug || spin >= 0;
+    int64_t qts = 0, kts = 0, vts = 0;
+    auto qc = packed ? q.contiguous() : token_rows(q, qts);
+    auto kc = packed ? k.contiguous() : token_rows(k, kts);
+    auto vc = packed ? v.contiguous() : token_rows(v, vts);
     auto gc = g.contiguous();
     auto bc = beta.contiguous();
     const int64_t B = qc.size(0), T = qc.size(1), HQK = qc.size(2), DK = qc.size(3);
@@ -83,7 +106,7 @@ std::vector<at::Tensor> chunk_prefill_impl(const at::Tensor& q, const at::Tensor
         N = cu32.numel() - 1;
     }
 
-    auto o = at::empty_like(vc);
+    auto o = at::empty({B, T, HV, DV}, vc.options());
     auto sf = at::empty({N, HV, DK, DV}, vc.options().dtype(at::kFloat));
     const float* s0p = nullptr;
     at::Tensor s0c;
@@ -116,24 +139,24 @@ std::vector<at::Tensor> chunk_prefill_impl(const at::Tensor& q, const at::Tensor
                                           s0p, sf.data_ptr<float>(), (int)B, (int)T, (int)HV,
                                           (int)HQK, ws.data_ptr(), ws_bytes, current_stream(),
                                           (unsigned)spin);
-    } else if (qk_l2norm) {
-        err = deltanet_chunk_prefill_l2norm(
-            qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr<float>(), bc.data_ptr<float>(),
-            o.data_ptr(), s0p, sf.data_ptr<float>(),
-            cu_seqlens.has_value() ? cu32.data_ptr<int32_t>() : nullptr, (int)N, (int)B, (int)T,
-            (int)HV, (int)HQK, ws.data_ptr(), ws_bytes, current_stream());
-    } else if (cu_seqlens.has_value()) {
-        err = deltanet_chunk_prefill_varlen(
-            qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr<float>(), bc.data_ptr<float>(),
-            o.data_ptr(), s0p, sf.data_ptr<float>(), cu32.data_ptr<int32_t>(), (int)N, (int)T,
-            (int)HV, (int)HQK, (int)DK, (int)DV, kChunk, ws.data_ptr(), ws_bytes,
-            current_stream(), debug ? 1 : 0);
+    } else if (debug) {
+        err = cu_seqlens.has_value()
+                  ? deltanet_chunk_prefill_varlen(
+                        qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr<float>(),
+                        bc.data_ptr<float>(), o.data_ptr(), s0p, sf.data_ptr<float>(),
+                        cu32.data_ptr<int32_t>(), (int)N, (int)T, (int)HV, (int)HQK, (int)DK,
+                        (int)DV, kChunk, ws.data_ptr(), ws_bytes, current_stream(), 1)
+                  : deltanet_chunk_prefill(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                                           gc.data_ptr<float>(), bc.data_ptr<float>(),
+                                           o.data_ptr(), s0p, sf.data_ptr<float>(), (int)B,
+                                           (int)T, (int)HV, (int)HQK, (int)DK, (int)DV, kChunk,
+                                           ws.data_ptr(), ws_bytes, current_stream(), 1);
     } else {
-        err = deltanet_chunk_prefill(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(),
-                                     gc.data_ptr<float>(), bc.data_ptr<float>(), o.data_ptr(), s0p,
-                                     sf.data_ptr<float>(), (int)B, (int)T, (int)HV, (int)HQK,
-                                     (int)DK, (int)DV, kChunk, ws.data_ptr(), ws_bytes,
-                                     current_stream(), debug ? 1 : 0);
+        err = deltanet_chunk_prefill_strided(
+            qc.data_ptr(), qts, kc.data_ptr(), kts, vc.data_ptr(), vts, gc.data_ptr<float>(),
+            bc.data_ptr<float>(), o.data_ptr(), s0p, sf.data_ptr<float>(),
+            cu_seqlens.has_value() ? cu32.data_ptr<int32_t>() : nullptr, (int)N, (int)B, (int)T,
+            (int)HV, (int)HQK, qk_l2norm ? 1 : 0, ws.data_ptr(), ws_bytes, current_stream());
     }
     check_hip(err, "deltanet_chunk_prefill");
     if (checked || spin >= 0) {
@@ -265,25 +288,27 @@ std::vector<at::Tensor> chunk_prefill_norm(at::Tensor q, at::Tensor k, at::Tenso
     return {y, sf};
 }
 
-at::Tensor recurrent_step(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor g,
-                          at::Tensor beta, at::Tensor state, bool qk_l2norm) {
+namespace {
+// Decode on `state_in` (undefined: zeros) into `state_out`, which may be it
+at::Tensor recurrent_impl(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                          const at::Tensor& g, const at::Tensor& beta, const at::Tensor& state_in,
+                          at::Tensor& state_out, bool qk_l2norm) {
     TORCH_CHECK(q.is_cuda() && k.is_cuda() && v.is_cuda() && g.is_cuda() && beta.is_cuda() &&
-                    state.is_cuda(),
+                    (!state_in.defined() || state_in.is_cuda()),
                 "all inputs must be CUDA tensors");
     TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 &&
                     v.scalar_type() == at::kBFloat16,
                 "q/k/v must be bf16");
     TORCH_CHECK(g.scalar_type() == at::kFloat && beta.scalar_type() == at::kFloat &&
-                    state.scalar_type() == at::kFloat,
+                    (!state_in.defined() || state_in.scalar_type() == at::kFloat),
                 "g/beta/state must be fp32");
     TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && g.dim() == 3 && beta.dim() == 3 &&
-                    state.dim() == 4,
+                    (!state_in.defined() || state_in.dim() == 4),
                 "bad ranks");
-    TORCH_CHECK(state.is_contiguous(), "state is updated in place and must be contiguous");
+    TORCH_CHECK(!state_in.defined() || state_in.is_contiguous(),
+                "state is updated in place and must be contiguous");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-    auto qc = q.contiguous();
-    auto kc = k.contiguous();
-    auto vc = v.contiguous();
+    const at::Tensor qc = head_rows(q), kc = head_rows(k), vc = head_rows(v);
     auto gc = g.contiguous();
     auto bc = beta.contiguous();
     const int64_t B = qc.size(0), T = qc.size(1), HQK = qc.size(2), DK = qc.size(3);
@@ -293,16 +318,45 @@ at::Tensor recurrent_step(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor g
                     gc.size(2) == HV && bc.sizes() == gc.sizes(),
                 "batch/time/head mismatch");
     TORCH_CHECK(HV % HQK == 0, "HV must be a multiple of HQK");
-    TORCH_CHECK(state.size(0) == B && state.size(1) == HV && state.size(2) == DK &&
-                    state.size(3) == DV,
+    TORCH_CHECK(!state_in.defined() || (state_in.size(0) == B && state_in.size(1) == HV &&
+                                        state_in.size(2) == DK && state_in.size(3) == DV),
                 "state must be [B, HV, DK, DV]");
-    auto o = at::empty_like(vc);
-    auto step = qk_l2norm ? deltanet_recurrent_step_l2norm : deltanet_recurrent_step;
-    check_hip(step(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr<float>(),
-                   bc.data_ptr<float>(), o.data_ptr(), state.data_ptr<float>(), (int)B, (int)T,
-                   (int)HV, (int)HQK, (int)DK, (int)DV, current_stream()),
+    TORCH_CHECK(DK == 128 && DV == 128, "only DK = DV = 128 is supported");
+    auto o = at::empty({B, T, HV, DV}, vc.options());
+    if (!state_out.defined()) {
+        state_out = at::empty({B, HV, DK, DV}, gc.options());
+        if (T == 0) {   // no token: the state as it was
+            if (state_in.defined()) state_out.copy_(state_in);
+            else state_out.zero_();
+        }
+    }
+    const at::Tensor& from = T == 0 ? state_out : state_in;
+    auto batch = [&](const at::Tensor& x) { return B > 1 ? x.stride(0) : 0; };
+    auto token = [&](const at::Tensor& x) { return T > 1 ? x.stride(1) : 0; };
+    check_hip(deltanet_recurrent_step_strided(
+                  qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr<float>(),
+                  bc.data_ptr<float>(), o.data_ptr(),
+                  from.defined() ? from.data_ptr<float>() : nullptr,
+                  state_out.data_ptr<float>(), (int)B, (int)T, (int)HV, (int)HQK, batch(qc),
+                  token(qc), batch(kc), token(kc), batch(vc), token(vc), qk_l2norm ? 1 : 0,
+                  current_stream()),
               "deltanet_recurrent_step");
     return o;
+}
+}  // namespace
+
+at::Tensor recurrent_step(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor g,
+                          at::Tensor beta, at::Tensor state, bool qk_l2norm) {
+    return recurrent_impl(q, k, v, g, beta, state, state, qk_l2norm);
+}
+
+// The same into a new state: returns [o, state]; state0 None is zeros.
+std::vector<at::Tensor> recurrent_step_new(at::Tensor q, at::Tensor k, at::Tensor v,
+                                           at::Tensor g, at::Tensor beta,
+                                           std::optional<at::Tensor> state0, bool qk_l2norm) {
+    at::Tensor s;
+    auto o = recurrent_impl(q, k, v, g, beta, state0 ? *state0 : at::Tensor(), s, qk_l2norm);
+    return {o, s};
 }
 
 at::Tensor gated_rmsnorm(at::Tensor x, at::Tensor z, at::Tensor weight, double eps) {
@@ -487,6 +541,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("recurrent_step", &recurrent_step,
           "recurrent gated delta rule (decode), state updated in place; returns o", "q"_a, "k"_a,
           "v"_a, "g"_a, "beta"_a, "state"_a, pybind11::kw_only(), "qk_l2norm"_a = false);
+    m.def("recurrent_step_new", &recurrent_step_new,
+          "recurrent_step into a new state; state0 None: zeros; returns [o, state]", "q"_a, "k"_a,
+          "v"_a, "g"_a, "beta"_a, "state0"_a = std::nullopt, pybind11::kw_only(),
+          "qk_l2norm"_a = false);
     m.def("chunk_prefill_fused", &chunk_prefill_fused,
           "prefill on raw inputs (q/k L2 norm, gates, dtype conversions fused); state updated "
           "in place; returns o",

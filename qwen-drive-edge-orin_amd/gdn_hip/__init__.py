@@ -13,6 +13,7 @@ The compiled pieces live next to this file:
   chunk_prefill_debug(...)  -> [o, final_state, T, A, cumsum_g, T_post_leaf, M, S_chunk]
   recurrent_step(q, k, v, g, beta, state, *, qk_l2norm=False) -> o
                                                         (state updated in place)
+  recurrent_step_new(q, k, v, g, beta, state0=None, *, qk_l2norm=False) -> [o, state]
   chunk_prefill_norm(q, k, v, g, beta, z, weight, s0=None, *, eps=1e-6, checked=False,
                      fused=False)
                           -> [gated_rmsnorm(o, z, weight), final_state]
@@ -82,6 +83,10 @@ def chunk_prefill_fused(q, k, v, a, b, A_log, dt_bias, state):
 
 def recurrent_step(q, k, v, g, beta, state, *, qk_l2norm=False):
     return load().recurrent_step(q, k, v, g, beta, state, qk_l2norm=qk_l2norm)
+
+
+def recurrent_step_new(q, k, v, g, beta, state0=None, *, qk_l2norm=False):
+    return load().recurrent_step_new(q, k, v, g, beta, state0, qk_l2norm=qk_l2norm)
 
 
 def gated_rmsnorm(x, z, weight, eps=1e-6):

@@ -60,6 +60,11 @@ _PROTOS = {
                                 [hipStream_t]),
     "deltanet_recurrent_step_l2norm": (hipError_t, [vp, vp, vp, fp, fp, vp, fp] + [c_int] * 6 +
                                        [hipStream_t]),
+    "deltanet_recurrent_step_strided": (hipError_t, [vp, vp, vp, fp, fp, vp, fp, fp] +
+                                        [c_int] * 4 + [c_int64] * 6 + [c_int, hipStream_t]),
+    "deltanet_chunk_prefill_strided": (hipError_t, [vp, c_int64, vp, c_int64, vp, c_int64, fp, fp,
+                                                    vp, fp, fp, i32p] + [c_int] * 6 +
+                                       [vp, c_size_t, hipStream_t]),
     "deltanet_prefill_kernel_count": (c_int, []),
     "deltanet_prefill_kernel_name": (ct.c_char_p, [c_int]),
     "deltanet_chunk_prefill_timed": (hipError_t, [vp, vp, vp, fp, fp, vp, fp, fp] + [c_int] * 7 +

@@ -77,8 +77,8 @@ def _prepare(q, k, v, g, beta, scale, use_qk_l2norm_in_kernel, kernel_norm=False
         q, k = _l2norm(q), _l2norm(k)
     if custom_scale:
         q = q.float() * (float(scale) / _KERNEL_SCALE)   # the kernels scale q by 1/sqrt(128)
-    return (q.to(bf).contiguous(), k.to(bf).contiguous(), v.to(bf).contiguous(),
-            g.float().contiguous(), beta.float().contiguous(), HV, in_kernel)
+    # q, k and v keep their strides: the ops read slices of one buffer in place
+    return q.to(bf), k.to(bf), v.to(bf), g.float(), beta.float(), HV, in_kernel
 
 
 def chunk_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None,
@@ -119,10 +119,6 @@ def recurrent_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None,
         raise NotImplementedError("recurrent_gated_delta_rule takes no cu_seqlens here")
     q, k, v, g, beta, HV, norm = _prepare(q, k, v, g, beta, scale, use_qk_l2norm_in_kernel,
                                           kernel_norm=True)
-    B = q.shape[0]
-    if initial_state is None:
-        state = torch.zeros(B, HV, _D, _D, dtype=torch.float32, device=q.device)
-    else:
-        state = initial_state.float().clone().contiguous()
-    o = gdn_hip.recurrent_step(q, k, v, g, beta, state, qk_l2norm=norm)
+    s0 = None if initial_state is None else initial_state.float().contiguous()
+    o, state = gdn_hip.recurrent_step_new(q, k, v, g, beta, s0, qk_l2norm=norm)
     return o.to(out_dtype), (state if output_final_state else None)

@@ -1,0 +1,66 @@
+"""q, k and v read where they lie (slices of one buffer, transposes, expanded
+rows, odd offsets) and the decode step into a new state: bitwise what the same
+values give from packed tensors and from the in-place step."""
+import pytest
+import torch
+
+import gdn_cases as gc
+
+pytestmark = pytest.mark.gpu
+
+# forms of one [B, T, H, 128] tensor with the same values
+FORMS = {
+    "slice": lambda x: torch.cat([x.flatten(2), x.flatten(2)], 2)[..., :x.shape[2] * 128]
+    .unflatten(2, (x.shape[2], 128)),
+    "odd_offset": lambda x: torch.cat([x.flatten()[:1], x.flatten()])[1:].view(x.shape),
+    "odd_stride": lambda x: torch.nn.functional.pad(x.flatten(2), (0, 3))[..., :x.shape[2] * 128]
+    .unflatten(2, (x.shape[2], 128)),
+    "tokens_first": lambda x: x.transpose(0, 1).contiguous().transpose(0, 1),
+    "heads_first": lambda x: x.transpose(1, 2).contiguous().transpose(1, 2),
+    "batch_gap": lambda x: torch.cat([x, x[:, :1]], 1)[:, :x.shape[1]],
+    "wide_elements": lambda x: torch.stack([x, x], -1)[..., 0],
+}
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("B,T,HK,HV", [(1, 77, 2, 4), (2, 130, 4, 4), (3, 1, 1, 2)])
+def test_prefill_strided(ops, dev, form, B, T, HK, HV):
+    q, k, v, g, beta, s0 = [t.to(dev) for t in gc.make_gdn_inputs(7, B=B, T=T, HK=HK, HV=HV,
+                                                                  g_shift=2.0)]
+    f = FORMS[form]
+    print(f"[strided] prefill {form} B={B} T={T} HK={HK} HV={HV}", flush=True)
+    for norm in (False, True):
+        o_ref, s_ref = ops.chunk_prefill(q, k, v, g, beta, s0, qk_l2norm=norm)
+        o, s = ops.chunk_prefill(f(q), f(k), f(v), g, beta, s0, qk_l2norm=norm)
+        assert o.is_contiguous() and torch.equal(o, o_ref) and torch.equal(s, s_ref)
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("B,T,HK,HV", [(1, 1, 2, 4), (3, 1, 2, 4), (2, 3, 1, 2)])
+def test_decode_strided_and_new_state(ops, dev, form, B, T, HK, HV):
+    q, k, v, g, beta, s0 = [t.to(dev) for t in gc.make_gdn_inputs(9, B=B, T=T, HK=HK, HV=HV,
+                                                                  g_shift=2.0)]
+    f = FORMS[form]
+    print(f"[strided] decode {form} B={B} T={T} HK={HK} HV={HV}", flush=True)
+    for norm in (False, True):
+        s_ref = s0.clone()
+        o_ref = ops.recurrent_step(q, k, v, g, beta, s_ref, qk_l2norm=norm)
+        s_in = s0.clone()
+        o = ops.recurrent_step(f(q), f(k), f(v), g, beta, s_in, qk_l2norm=norm)
+        assert torch.equal(o, o_ref) and torch.equal(s_in, s_ref)
+        keep = s0.clone()
+        o, s = ops.recurrent_step_new(f(q), f(k), f(v), g, beta, keep, qk_l2norm=norm)
+        assert torch.equal(o, o_ref) and torch.equal(s, s_ref) and torch.equal(keep, s0)
+        s_ref = torch.zeros_like(s0)
+        o_ref = ops.recurrent_step(q, k, v, g, beta, s_ref, qk_l2norm=norm)
+        o, s = ops.recurrent_step_new(f(q), f(k), f(v), g, beta, None, qk_l2norm=norm)
+        assert torch.equal(o, o_ref) and torch.equal(s, s_ref)
+
+
+def test_decode_new_state_without_tokens(ops, dev):
+    q, k, v, g, beta, s0 = [t.to(dev) for t in gc.make_gdn_inputs(9, B=2, T=1, HK=2, HV=4)]
+    e = [t[:, :0] for t in (q, k, v, g, beta)]
+    o, s = ops.recurrent_step_new(*e, s0)
+    assert o.shape == (2, 0, 4, 128) and torch.equal(s, s0) and s.data_ptr() != s0.data_ptr()
+    with pytest.raises(RuntimeError):
+        ops.recurrent_step_new(*[t[:0] for t in e], s0[:0])
