@@ -359,6 +359,41 @@ std::vector<at::Tensor> recurrent_step_new(at::Tensor q, at::Tensor k, at::Tenso
     return {o, s};
 }
 
+// The adapter's decode call in its ordinary form: everything on one device,
+// bf16 q, k, v of matching shapes, fp32 g, beta and state.  Returns None for
+// anything else, which the adapter then converts or refuses itself.  One call
+// here stands for ~30 attribute reads in Python (a one-user layer step with
+// conv and norm: 25.8 -> 21.5 us, bound by the host).
+py::object recurrent_ordinary(py::handle q_, py::handle k_, py::handle v_, py::handle g_,
+                              py::handle beta_, py::handle s_, bool qk_l2norm) {
+    for (py::handle h : {q_, k_, v_, g_, beta_})
+        if (!THPVariable_Check(h.ptr())) return py::none();
+    const bool zeros = s_.is_none();
+    if (!zeros && !THPVariable_Check(s_.ptr())) return py::none();
+    const at::Tensor &q = THPVariable_Unpack(q_.ptr()), &k = THPVariable_Unpack(k_.ptr()),
+                     &v = THPVariable_Unpack(v_.ptr()), &g = THPVariable_Unpack(g_.ptr()),
+                     &beta = THPVariable_Unpack(beta_.ptr());
+    const at::Tensor s = zeros ? at::Tensor() : THPVariable_Unpack(s_.ptr());
+    if (!q.is_cuda() || q.dim() != 4 || v.dim() != 4 || k.sizes() != q.sizes()) return py::none();
+    const int64_t B = q.size(0), T = q.size(1), HQ = q.size(2), HV = v.size(2);
+    if (B < 1 || T < 1 || HQ < 1 || q.size(3) != 128 || v.size(3) != 128 || v.size(0) != B ||
+        v.size(1) != T || HV < 1 || HV % HQ != 0)
+        return py::none();
+    for (const at::Tensor* t : {&q, &k, &v})
+        if (t->scalar_type() != at::kBFloat16 || t->device() != q.device()) return py::none();
+    for (const at::Tensor* t : {&g, &beta})
+        if (t->scalar_type() != at::kFloat || t->device() != q.device() || t->dim() != 3 ||
+            t->size(0) != B || t->size(1) != T || t->size(2) != HV)
+            return py::none();
+    if (!zeros && (s.scalar_type() != at::kFloat || s.device() != q.device() || s.dim() != 4 ||
+                   s.size(0) != B || s.size(1) != HV || s.size(2) != 128 || s.size(3) != 128 ||
+                   !s.is_contiguous()))
+        return py::none();
+    at::Tensor out;
+    at::Tensor o = recurrent_impl(q, k, v, g, beta, s, out, qk_l2norm);
+    return py::make_tuple(o, out);
+}
+
 at::Tensor gated_rmsnorm(at::Tensor x, at::Tensor z, at::Tensor weight, double eps) {
     TORCH_CHECK(x.is_cuda() && z.is_cuda() && weight.is_cuda(), "all inputs must be CUDA tensors");
     TORCH_CHECK(x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf,
@@ -545,6 +580,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "recurrent_step into a new state; state0 None: zeros; returns [o, state]", "q"_a, "k"_a,
           "v"_a, "g"_a, "beta"_a, "state0"_a = std::nullopt, pybind11::kw_only(),
           "qk_l2norm"_a = false);
+    m.def("_recurrent_ordinary", &recurrent_ordinary,
+          "recurrent_step_new for ordinary arguments, None for any others");
     m.def("chunk_prefill_fused", &chunk_prefill_fused,
           "prefill on raw inputs (q/k L2 norm, gates, dtype conversions fused); state updated "
           "in place; returns o",

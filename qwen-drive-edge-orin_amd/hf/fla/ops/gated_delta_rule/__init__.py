@@ -112,8 +112,11 @@ def recurrent_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None,
     """Token-by-token gated delta rule (decode).  Returns ``(o, final_state)``
     with o in q's dtype (modeling_qwen3_5.py:379); the caller's initial_state
     is not modified."""
-    import torch
-
+    if scale is None and cu_seqlens is None:
+        r = gdn_hip.load()._recurrent_ordinary(q, k, v, g, beta, initial_state,
+                                               bool(use_qk_l2norm_in_kernel))
+        if r is not None:
+            return r if output_final_state else (r[0], None)
     out_dtype = q.dtype
     if cu_seqlens is not None:
         raise NotImplementedError("recurrent_gated_delta_rule takes no cu_seqlens here")
