@@ -356,11 +356,12 @@ __device__ bool locate_chunk(const int32_t* cu, int N, int T, int total, int cid
 // each other): after the prep's 30 MB of workspace that write-back held the
 // scan back ~5 us, with these stores ~1.3 us.  Non-temporal stores (kNt)
 // avoid the write-back too, but the lines then come back from HBM: slower
-// while a call's records fit the 256 MB memory-side cache (T1141 HV32
-// 37.2 -> 40.8 us; up to 233 MB of workspace 3-10 % slower), faster once
+// while a call's records fit the 256 MB memory-side cache beside its inputs
+// and o (T1141 HV32 37.2 -> 40.8 us; 100 MB written 3 % slower), faster once
 // they do not, when the scan reads them from HBM either way and the written
-// lines only push older ones out (276 to 686 MB of workspace: 3.3-5.5 %
-// faster); the launcher picks them above kNtWorkspaceBytes.  The prep never
+// lines only push older ones out (214 MB written, 2 x 3200 tokens HV32 HK32:
+// 158.0 -> 153.9 us; 209 to 512 MB 3.3-5.5 %; 176 MB the same).  The launcher
+// picks them above kNtRecordBytes written.  The prep never
 // waits for these stores.  The scan's o and state
 // stores stay plain: a wave's later loads complete only after its earlier
 // stores, and waiting behind write-through stores slowed the output waves by
@@ -369,7 +370,7 @@ __device__ bool locate_chunk(const int32_t* cu, int N, int T, int total, int cid
 // which the compiler inserts after its own stores but cannot see inside an
 // asm statement, so the 16-byte form carries its own s_nop.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-constexpr size_t kNtWorkspaceBytes = size_t(256) << 20;
+constexpr size_t kNtRecordBytes = size_t(192) << 20;
 template <bool kNt = false, typename V>
 __device__ __forceinline__ void st_through(V* p, const V& v) {
     static_assert(sizeof(V) == 4 || sizeof(V) == 8 || sizeof(V) == 16, "4, 8 or 16 bytes");
@@ -2916,7 +2917,9 @@ hipError_t launch_prefill(PrepIn in, int raw, void* o, const float* s0, float* s
         const size_t grid = std::max<size_t>(groups * 8 * rep, 1);
         // records that cannot stay in the memory-side cache go out
         // non-temporally (see st_through)
-        const bool nt = !dump_debug && need > kNtWorkspaceBytes;
+        const size_t written = nch_bound * HV * (3 * kTriBytes + kWBytes + kGateBytes) +
+                               nch_bound * HK * (kQBytes + kKTBytes);
+        const bool nt = !dump_debug && written > kNtRecordBytes;
         auto kern = raw == 1 ? (nt ? gdn_prep_kernel<false, 1, true> : gdn_prep_kernel<false, 1>)
                     : raw == 2 ? (nt ? gdn_prep_kernel<false, 2, true> : gdn_prep_kernel<false, 2>)
                     : dump_debug ? gdn_prep_kernel<true, 0>
