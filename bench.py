@@ -195,7 +195,8 @@ def bench_varlen(ops, dev, steps, warmup):
     algo = _bytes(q, k, v, g, beta, s0) + _bytes(v) + _bytes(s0)
     out = dict(ms=ms, tflops=flops / ms / 1e9, gbs=algo / ms / 1e6, tokens=total)
     # the same call with each scan instance forced (deltanet_chunk_prefill_cols):
-    # 16 value columns per work-group, and the paired 32 the library picks here
+    # 16 value columns per work-group, and the paired 32 (the library picks the
+    # wide 64-column instance here)
     import ctypes as ct
     from gdn_hip import capi
 
@@ -429,8 +430,9 @@ def bench_twolevel(ops, dev, reps=10):
 
         def groups(pairs):
             # the library's scan instance: 16-column groups while they fit on
-            # the CUs at once, the paired 32-column instance beyond
-            per = 8 if pairs * 8 <= cus else 4
+            # the CUs at once, then the paired 32-column and the wide
+            # 64-column instance
+            per = 8 if pairs * 8 <= cus else 4 if pairs * 4 <= cus else 2
             return -(-pairs // 8) * 8 * per
 
         nseg = sum(min(segs, c) if c else 1 for c in nch)

@@ -60,8 +60,9 @@ hipError_t deltanet_chunk_prefill_spin(const void* q, const void* k, const void*
  * with the scan instance chosen by the caller: slice_cols 16 runs one scan
  * work-group per 16 value columns of a (sequence, head), 32 the paired
  * instance with one per 32 columns, 128 the wide instance (the whole head: two
- * work-groups of 64 columns), 0 the library's own choice (the narrowest whose
- * groups fit on the device's CUs at once, else the wide one).  All give
+ * work-groups of 64 columns), 0 the library's own choice (16 while its
+ * groups fit on the device's CUs at once, then 32, then the wide one; the wide
+ * one instead of 32 above 48 heads whose operands come from beyond an L2).  All give
  * bitwise the same o and final state; the wide instance has no bounded waits.  cu_seqlens NULL: num_seqs sequences of
  * T tokens; otherwise a device array [num_seqs + 1] and T the total token
  * count.  spin_limit 0 keeps the library's bounded-wait limit, otherwise as in

@@ -38,7 +38,9 @@
 //         (deltanet_prefill_status).  Once a call's 16-column groups would
 //         outnumber the CUs, a paired instance gives each work-group 32
 //         columns as two 16-column halves sharing the chunk operands
-//         (gdn_scan2_kernel; bitwise the same results).
+//         (gdn_scan2_kernel), and once those would too, a wide instance 64
+//         columns, one compute wave per 16 (gdn_scan_wide_kernel; bitwise the
+//         same results).
 //
 // Rounding budget (checked against an fp64 emulation of each operand class):
 // W and S rounded to fp16 for V_n change the final state by < 1e-4 relative;
@@ -2427,6 +2429,12 @@ __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan2_kernel(ScanArgs a) 
 // by the loaders (as 32-byte pieces from the compute waves it took 0.4 us a
 // step).  The arithmetic per 16 columns is the 16-column instance's,
 // operation for operation (o and the final state are bitwise the same).
+//
+// Bound by the loads where the records come from beyond L2 (75 KB a step at
+// ~36 B/ns per CU: 2.1 us, the same without the compute), by the compute
+// waves' issue and LDS reads where they are in cache (1.6 us, the same without
+// the loads).  8 packed prompts of 19,861 tokens, HV 32: the scan 285 us with
+// the paired instance, 187 with this one; 4 x 1141 tokens 59 and 41.
 // ---------------------------------------------------------------------------
 constexpr int kWideCols = 64;
 constexpr int kWideSlices = kWideCols / kSliceCols;   // 4, one per compute wave
@@ -2486,26 +2494,16 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
 #pragma unroll
         for (int f = 0; f < 4; ++f) lds_dma16(sp + f * 64, dp + f * 64);
     };
-    // The two groups of a head (one L2) take its records in opposite orders:
-    // each then finds the half that the other brought in L2.
     auto issue_a = [&](int cc) {
         const int c = min(cc, x.nch - 1);
         StageWideA& st = sm.a[cc & 1];
         const size_t ck = (size_t)(x.chunk0 + c), ch = ck * a.HV + x.hv, kq = ck * a.HK + x.hk;
-        auto tri = [&] {   // fragments 3 j .. 3 j + 2 of hi and lo in a row
-            const half8* src = (j < 2 ? a.ws.TI : a.ws.TIlo) + (ch * kTri + 3 * (j & 1)) * 64 + lane;
+        // fragments 3 j .. 3 j + 2 of hi and lo in a row
+        const half8* tsrc = (j < 2 ? a.ws.TI : a.ws.TIlo) + (ch * kTri + 3 * (j & 1)) * 64 + lane;
 #pragma unroll
-            for (int f = 0; f < 3; ++f) lds_dma16(src + f * 64, &st.T[3 * j + f][0]);
-        };
-        if (x.sl == 0) {
-            tri();
-            four(a.ws.W, ch, st.W);
-            four(a.ws.Q, kq, st.Q);
-        } else {
-            four(a.ws.Q, kq, st.Q);
-            four(a.ws.W, ch, st.W);
-            tri();
-        }
+        for (int f = 0; f < 3; ++f) lds_dma16(tsrc + f * 64, &st.T[3 * j + f][0]);
+        four(a.ws.W, ch, st.W);
+        four(a.ws.Q, kq, st.Q);
         if (j == kWideLoaders - 1)
             lds_dma16(a.ws.gates + ch * (kGateBytes / 4) + 4 * lane, &st.gates[0]);
         const int t0 = x.tok_base + c * kChunk, rows = min(kChunk, x.len - c * kChunk);
@@ -2521,13 +2519,14 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
         const int c = min(cc, x.nch - 1);
         StageWideB& st = sm.b[cc & 1];
         const size_t ck = (size_t)(x.chunk0 + c), ch = ck * a.HV + x.hv;
-        if (x.sl == 0) four(a.ws.KT, ck * a.HK + x.hk, st.KT);
+        four(a.ws.KT, ck * a.HK + x.hk, st.KT);
         const half8* src = a.ws.M + (ch * kTri + j) * 64 + lane;
         lds_dma16(src, &st.M[j][0]);
         if (j < kTri - kWideLoaders) lds_dma16(src + kWideLoaders * 64, &st.M[j + kWideLoaders][0]);
-        if (x.sl != 0) four(a.ws.KT, ck * a.HK + x.hk, st.KT);
     };
-    // O of chunk c, rows 16 j .. + 15.  The reads and their wait are one asm
+    // O of chunk c, rows 16 j .. + 15, whole lines that nothing here reads
+    // again: non-temporal (2 x 3200 tokens HV32 HK32 153.2 -> 148.1 us, 4 x
+    // 1141 HV32 75.0 -> 70.9).  The reads and their wait are one asm
     // block: the compiler would place a wait for every direct-to-LDS load in
     // front of an LDS read of its own.
     auto store_o = [&](int c) {
@@ -2544,9 +2543,11 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
         for (int i = 0; i < 2; ++i) {
             const int r = 16 * j + 8 * i + (lane >> 3), p = (lane ^ r) & 7;
             if (r < rows)
-                *reinterpret_cast<u32x4*>(
-                    a.o + ((size_t)(x.tok_base + c * kChunk + r) * a.HV + x.hv) * kDV +
-                    kWideCols * x.sl + 8 * p) = i ? v1 : v0;
+                __builtin_nontemporal_store(
+                    i ? v1 : v0,
+                    reinterpret_cast<u32x4*>(
+                        a.o + ((size_t)(x.tok_base + c * kChunk + r) * a.HV + x.hv) * kDV +
+                        kWideCols * x.sl + 8 * p));
         }
     };
     if (x.nch <= 0) return;
@@ -2863,14 +2864,21 @@ int device_cus() {
 // Scan instance (value columns per work-group): 16-column groups while they
 // fit on the CUs at once (one group per CU), the paired 32-column groups once
 // they would run in rounds (then the halves' shared operands halve the
-// rounds), the wide 64-column groups once the paired ones would.  cols forces
-// one (diagnostics); the debug dump and the norm epilogue exist in the
-// 16-column instance only.
-int scan_cols(int cols, int N, int HV, int dump_debug, bool norm) {
+// rounds), the wide 64-column groups once the paired ones would (paired and
+// wide, 3 x 1141 tokens HV32: 74.7 and 59.8 us; 6 x 256: 43.9 and 35.2; 8
+// packed prompts, 19,861 tokens: 430 and 340), or, with more than 48 heads,
+// where each group's operands come from beyond its L2 (`far`: every head has
+// its own Q and K^T, or the records outgrow the memory-side cache) and the
+// wide groups' half as many fetches count (2 x 2000 tokens HV32 HK32: 94.7
+// and 86.6; 2 x 4096 HV32 HK16: 171 and 166; but 2 x 1141 HV32 HK16 45.5 and
+// 49, and 48 heads 117.5 and 118.7).  cols forces one (diagnostics); the debug
+// dump and the norm epilogue exist in the 16-column instance only.
+int scan_cols(int cols, int N, int HV, int dump_debug, bool norm, bool far) {
     if (cols) return cols;
     if (dump_debug || norm) return kSliceCols;
     const long long heads = (long long)N * HV, cus = device_cus();
     if (heads * kSlicesPerHead <= cus) return kSliceCols;
+    if (far && heads * 16 > cus * 3) return kWideCols;
     return heads * kPairsPerHead <= cus ? kPairCols : kWideCols;
 }
 
@@ -2880,7 +2888,11 @@ hipError_t launch_prefill(PrepIn in, int raw, void* o, const float* s0, float* s
                           hipStream_t stream, int dump_debug, hipEvent_t* ev = nullptr,
                           int only = -1, unsigned spin = kDefaultSpin,
                           const NormIn* norm = nullptr, int cols = 0) {
-    const int width = scan_cols(cols, N, HV, dump_debug, norm != nullptr);
+    // records written non-temporally: see st_through
+    const size_t written = nch_bound * HV * (3 * kTriBytes + kWBytes + kGateBytes) +
+                           nch_bound * HK * (kQBytes + kKTBytes);
+    const bool nt = !dump_debug && written > kNtRecordBytes;
+    const int width = scan_cols(cols, N, HV, dump_debug, norm != nullptr, nt || HV == HK);
     if (width != kSliceCols && (dump_debug || norm)) return hipErrorInvalidValue;
     if (in.qts < 0) in.qts = HK * kDK;
     if (in.kts < 0) in.kts = HK * kDK;
@@ -2915,11 +2927,6 @@ hipError_t launch_prefill(PrepIn in, int raw, void* o, const float* s0, float* s
         const int rep = HV / HK;
         const size_t groups = (nch_bound * (size_t)HK + 7) / 8;
         const size_t grid = std::max<size_t>(groups * 8 * rep, 1);
-        // records that cannot stay in the memory-side cache go out
-        // non-temporally (see st_through)
-        const size_t written = nch_bound * HV * (3 * kTriBytes + kWBytes + kGateBytes) +
-                               nch_bound * HK * (kQBytes + kKTBytes);
-        const bool nt = !dump_debug && written > kNtRecordBytes;
         auto kern = raw == 1 ? (nt ? gdn_prep_kernel<false, 1, true> : gdn_prep_kernel<false, 1>)
                     : raw == 2 ? (nt ? gdn_prep_kernel<false, 2, true> : gdn_prep_kernel<false, 2>)
                     : dump_debug ? gdn_prep_kernel<true, 0>
@@ -3084,7 +3091,7 @@ extern "C" hipError_t deltanet_chunk_prefill_norm_fused(
     // The epilogue lives in the 16-column scan; where the plain prefill would
     // take the paired 32-column instance (more slice groups than CUs) the
     // two-kernel path runs instead.
-    if (scan_cols(0, B, HV, 0, false) != kSliceCols)
+    if (scan_cols(0, B, HV, 0, false, false) != kSliceCols)
         return prefill_then_norm(q, k, v, g, beta, z, norm_weight, eps, y, initial_state,
                                  final_state, B, T, HV, HQK, workspace, workspace_bytes, stream);
     const size_t nc = (size_t)B * ((T + kChunk - 1) / kChunk);

@@ -389,6 +389,7 @@ py::object recurrent_ordinary(py::handle q_, py::handle k_, py::handle v_, py::h
                    s.size(0) != B || s.size(1) != HV || s.size(2) != 128 || s.size(3) != 128 ||
                    !s.is_contiguous()))
         return py::none();
+    if (!zeros && s.requires_grad() && at::GradMode::is_enabled()) return py::none();
     at::Tensor out;
     at::Tensor o = recurrent_impl(q, k, v, g, beta, s, out, qk_l2norm);
     return py::make_tuple(o, out);

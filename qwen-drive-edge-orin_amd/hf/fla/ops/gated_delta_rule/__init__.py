@@ -123,5 +123,9 @@ def recurrent_gated_delta_rule(q, k, v, g, beta, scale=None, initial_state=None,
     q, k, v, g, beta, HV, norm = _prepare(q, k, v, g, beta, scale, use_qk_l2norm_in_kernel,
                                           kernel_norm=True)
     s0 = None if initial_state is None else initial_state.float().contiguous()
-    o, state = gdn_hip.recurrent_step_new(q, k, v, g, beta, s0, qk_l2norm=norm)
+    if s0 is not None and s0.requires_grad:   # autograd sees a copy of it, as ever
+        state = s0.clone()
+        o = gdn_hip.recurrent_step(q, k, v, g, beta, state, qk_l2norm=norm)
+    else:
+        o, state = gdn_hip.recurrent_step_new(q, k, v, g, beta, s0, qk_l2norm=norm)
     return o.to(out_dtype), (state if output_final_state else None)
