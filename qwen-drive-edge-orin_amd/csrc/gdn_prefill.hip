@@ -169,6 +169,11 @@ struct PrepIn {
 // ---------------------------------------------------------------------------
 // element helpers
 // ---------------------------------------------------------------------------
+// Elements to row t at stride ts (both non-negative): one 32 x 32-bit product
+__device__ __forceinline__ size_t row_at(int t, int ts) {
+    return (size_t)(uint32_t)t * (uint32_t)ts;
+}
+
 // A raw 16-bit input element as fp32 (kRaw 0/1: bf16, 2: fp16)
 template <int kRaw>
 __device__ inline float raw16(uint32_t bits) {
@@ -544,18 +549,18 @@ __global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(
     // K: thread tid holds piece tid % 16 of rows tid / 16 + 16 ii
     u32x4 raw[4];
     {
-        const uint16_t* base = k + (size_t)tok0 * in.kts + hk * kDK + 8 * (tid & 15);
+        const uint16_t* base = k + row_at(tok0, in.kts) + hk * kDK + 8 * (tid & 15);
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii) {
             const int r = min((tid >> 4) + 16 * ii, rows - 1);
-            raw[ii] = *reinterpret_cast<const u32x4*>(base + (size_t)r * in.kts);
+            raw[ii] = *reinterpret_cast<const u32x4*>(base + row_at(r, in.kts));
         }
     }
     // Q: wave w, lane (lg, lm) holds row 16 w + lm, dk 32 kb + 8 lg .. + 7
     u32x4 qr[4];
     {
         const uint16_t* qs =
-            q + (size_t)(tok0 + min(wave * 16 + lm, rows - 1)) * in.qts + hk * kDK + 8 * lg;
+            q + row_at(tok0 + min(wave * 16 + lm, rows - 1), in.qts) + hk * kDK + 8 * lg;
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) qr[kb] = *reinterpret_cast<const u32x4*>(qs + kb * 32);
     }
@@ -1083,7 +1088,7 @@ __device__ void run_loader(ScanSmem& sm, const ScanArgs& a, const Waiter& w, con
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int s = 64 * i + lane, r = min(s >> 1, rows - 1);
-            lds_dma16(a.in.v + (size_t)(t0 + r) * a.in.vts + x.hv * kDV + kSliceCols * x.sl + 8 * (s & 1),
+            lds_dma16(a.in.v + row_at(t0 + r, a.in.vts) + x.hv * kDV + kSliceCols * x.sl + 8 * (s & 1),
                       &st.V[64 * i]);
         }
         lds_dma16(a.ws.gates + ch_of(c) * (kGateBytes / 4) + 4 * lane, &st.gates[0]);
@@ -1947,7 +1952,7 @@ __device__ void run_loader2(ScanSmem2& sm, const ScanArgs& a, const Waiter& w, c
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int s = 64 * i + lane, r = min(s >> 1, rows - 1);
-                lds_dma16(a.in.v + (size_t)(t0 + r) * a.in.vts + x.hv * kDV + kPairCols * x.sl +
+                lds_dma16(a.in.v + row_at(t0 + r, a.in.vts) + x.hv * kDV + kPairCols * x.sl +
                               kSliceCols * h + 8 * (s & 1),
                           &sp.V[h][64 * i]);
             }
@@ -2510,7 +2515,7 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int r = 16 * j + 8 * i + (lane >> 3), p = (lane ^ r) & 7;   // slot 8 r + lane % 8
-            lds_dma16(a.in.v + (size_t)(t0 + min(r, rows - 1)) * a.in.vts + x.hv * kDV +
+            lds_dma16(a.in.v + row_at(t0 + min(r, rows - 1), a.in.vts) + x.hv * kDV +
                           kWideCols * x.sl + 8 * p,
                       &st.V[(16 * j + 8 * i) * 8]);
         }
