@@ -487,11 +487,11 @@ __global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(
     PrepIn in, const int32_t* __restrict__ cu, int N, int T, int total, int HV, int HK,
     int nch_bound, float scale, Workspace ws) {
     __shared__ PrepSmem sm;
-    // The kernel arguments (240 bytes) span four 64-byte lines, which the
+    // The kernel arguments (256 bytes) span four 64-byte lines, which the
     // scalar cache would otherwise fetch in three dependent round trips (each
-    // use waits before the branch that leads to the next): fields at most 32
-    // bytes apart, all requested together, cost one.
-    asm volatile("" ::"s"(in.q), "s"(in.A_log), "s"(in.kts), "s"(cu), "s"(nch_bound), "s"(ws.TIlo),
+    // use waits before the branch that leads to the next): a field of each,
+    // all requested together, cost one.
+    asm volatile("" ::"s"(in.q), "s"(in.A_log), "s"(cu), "s"(nch_bound), "s"(ws.TIlo),
                  "s"(ws.gates), "s"(ws.ncnt), "s"(ws.dbgT), "s"(ws.dbgM), "s"(ws.dbgS));
     const uint16_t* __restrict__ q = in.q;
     const uint16_t* __restrict__ k = in.k;
@@ -1782,10 +1782,10 @@ __device__ inline void scan_context(const ScanArgs& a, int pidx, int* seqsel, in
 template <int kRaw, bool kDbg, bool kNorm = false>
 __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan_kernel(ScanArgs a) {
     __shared__ ScanSmem sm;
-    // The kernel arguments (288 bytes) span five 64-byte lines, which the
-    // scalar cache would otherwise fetch in three dependent round trips:
-    // fields at most 32 bytes apart, all requested together, cost one.
-    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.in.vts), "s"(a.ws.M), "s"(a.ws.KT),
+    // The kernel arguments (304 bytes) span five 64-byte lines, which the
+    // scalar cache would otherwise fetch in three dependent round trips: a
+    // field of each, all requested together, cost one.
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
                  "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
                  "s"(a.spin));
     const int tid = threadIdx.x;
@@ -2370,7 +2370,7 @@ template <int kRaw>
 __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan2_kernel(ScanArgs a) {
     __shared__ ScanSmem2 sm;
     // kernel-argument lines requested together (as in gdn_scan_kernel)
-    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.in.vts), "s"(a.ws.M), "s"(a.ws.KT),
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
                  "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
                  "s"(a.spin));
     const int tid = threadIdx.x;
@@ -2816,7 +2816,7 @@ template <int kRaw>
 __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan_wide_kernel(ScanArgs a) {
     __shared__ ScanSmemWide sm;
     // kernel-argument lines requested together (as in gdn_scan_kernel)
-    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.in.vts), "s"(a.ws.M), "s"(a.ws.KT),
+    asm volatile("" ::"s"(a.in.q), "s"(a.in.beta), "s"(a.in.dt_bias), "s"(a.ws.M), "s"(a.ws.KT),
                  "s"(a.ws.dbgT), "s"(a.ws.dbgC), "s"(a.z), "s"(a.s0), "s"(a.N), "s"(a.HK),
                  "s"(a.spin));
     const int tid = threadIdx.x;
