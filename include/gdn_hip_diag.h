@@ -99,6 +99,11 @@ int deltanet_varlen_chunks_before(const int32_t* cu_seqlens, int num_seqs, int t
 int deltanet_varlen_locate_chunk(const int32_t* cu_seqlens, int num_seqs, int total_tokens,
                                  int cid, int nt, int32_t* seq_tok_rows);
 
+/* Element offset of batch b's token t, head h in packed q, k or v rows
+ * [B][T][heads][128] as the decode kernels form it (host only, the kernels'
+ * arithmetic): 64 bits, also where a batch's T tokens span 2^31 elements. */
+size_t deltanet_recurrent_row_offset(int T, int heads, int b, int t, int h);
+
 /* Two-level chunk-group scan (prototype for measurement; same results as
  * deltanet_chunk_prefill / _varlen to rounding).  Each sequence's chunks are
  * cut into `segments` chunk-aligned segments; pass 1 scans every segment

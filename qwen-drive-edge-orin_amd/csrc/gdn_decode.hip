@@ -50,9 +50,15 @@ static_assert(kRowGroups * kRowsPerThread == kDK && kRowGroups % 4 == 0, "row gr
 // state instead of two (a B=24 HV=32 layer step with conv and norm: 49.5 ->
 // 26 us).  Reading and writing one buffer is safe: a thread reads its
 // elements before it writes them, and no other thread touches them.
-struct DecStrides {
-    int qb, qt, kb, kt, vb, vt;   // elements
+struct DecStrides {   // elements; a batch's T tokens may span more than 31 bits
+    int64_t qb, kb, vb;
+    int qt, kt, vt;
 };
+
+// Elements in front of batch b's token t
+__host__ __device__ __forceinline__ size_t dec_row(int b, int64_t bs, int t, int ts) {
+    return (size_t)b * (size_t)bs + (size_t)t * (size_t)ts;
+}
 
 // kFrom: where the state comes from
 constexpr int kFromOut = 0, kFromIn = 1, kFromZero = 2;   // state_out itself, state_in, zeros
@@ -85,15 +91,15 @@ __global__ __launch_bounds__(kDecThreads) void gdn_recurrent_kernel(
     // (128..255), its four v columns, g and beta.  Token 0's are requested
     // before the state, so forming q and k needs only them; each later
     // token's are requested during the previous token's work.
-    const uint16_t* qk = tid < kDK ? q + (size_t)b * st.qb + (size_t)hk * kDK + tid
-                                   : k + (size_t)b * st.kb + (size_t)hk * kDK + tid - kDK;
+    const uint16_t* qk = tid < kDK ? q + dec_row(b, st.qb, 0, st.qt) + (size_t)hk * kDK + tid
+                                   : k + dec_row(b, st.kb, 0, st.kt) + (size_t)hk * kDK + tid - kDK;
     const int qkt = tid < kDK ? st.qt : st.kt;
-    const uint16_t* vp = v + (size_t)b * st.vb + (size_t)hv * kDV + c0 + 4 * cb;
+    const uint16_t* vp = v + dec_row(b, st.vb, 0, st.vt) + (size_t)hv * kDV + c0 + 4 * cb;
     float* qk_dst = tid < kDK ? qs + tid : ks + tid - kDK;
     auto load_token = [&](int t, uint16_t& qkr, uint2& vr, float& gr, float& br) {
         const size_t tk = (size_t)b * T + t;
-        qkr = qk[(size_t)t * qkt];
-        vr = *reinterpret_cast<const uint2*>(vp + (size_t)t * st.vt);
+        qkr = qk[dec_row(0, 0, t, qkt)];
+        vr = *reinterpret_cast<const uint2*>(vp + dec_row(0, 0, t, st.vt));
         gr = g[tk * HV + hv];
         br = beta[tk * HV + hv];
     };
@@ -219,9 +225,9 @@ hipError_t recurrent_launch(const void* q, const void* k, const void* v, const f
         const size_t tk = (size_t)b0 * T, so = (size_t)b0 * HV * kDK * kDV;
         hipLaunchKernelGGL(kern, dim3((unsigned)(kDecSplit * HV), (unsigned)std::min(B - b0, 65535)),
                            dim3(kDecThreads), 0, stream,
-                           static_cast<const uint16_t*>(q) + (size_t)b0 * st.qb,
-                           static_cast<const uint16_t*>(k) + (size_t)b0 * st.kb,
-                           static_cast<const uint16_t*>(v) + (size_t)b0 * st.vb, g + tk * HV,
+                           static_cast<const uint16_t*>(q) + dec_row(b0, st.qb, 0, st.qt),
+                           static_cast<const uint16_t*>(k) + dec_row(b0, st.kb, 0, st.kt),
+                           static_cast<const uint16_t*>(v) + dec_row(b0, st.vb, 0, st.vt), g + tk * HV,
                            beta + tk * HV, static_cast<uint16_t*>(o) + tk * HV * kDV,
                            state_in ? state_in + so : nullptr, state_out + so, T, HV, HV / HQK,
                            1.0f / sqrtf((float)kDK), st);
@@ -233,7 +239,7 @@ hipError_t recurrent_launch(const void* q, const void* k, const void* v, const f
 // q, k [B][T][HQK][DK] and v [B][T][HV][DV] without gaps
 DecStrides packed(int T, int HV, int HQK) {
     const int qt = HQK * kDK, vt = HV * kDV;
-    return DecStrides{T * qt, qt, T * qt, qt, T * vt, vt};
+    return DecStrides{(int64_t)T * qt, (int64_t)T * qt, (int64_t)T * vt, qt, qt, vt};
 }
 }  // namespace
 
@@ -270,7 +276,12 @@ extern "C" hipError_t deltanet_recurrent_step_strided(
         return hipErrorInvalidValue;
     }
     return recurrent_launch(q, k, v, g, beta, o, state_in, state_out, B, T, HV, HQK, kDK, kDV,
-                            DecStrides{(int)q_batch, (int)q_token, (int)k_batch, (int)k_token,
-                                       (int)v_batch, (int)v_token},
+                            DecStrides{q_batch, k_batch, v_batch, (int)q_token, (int)k_token,
+                                       (int)v_token},
                             stream, qk_l2norm != 0);
+}
+
+extern "C" size_t deltanet_recurrent_row_offset(int T, int heads, int b, int t, int h) {
+    const DecStrides st = packed(T, heads, heads);
+    return dec_row(b, st.vb, t, st.vt) + (size_t)h * kDV;
 }

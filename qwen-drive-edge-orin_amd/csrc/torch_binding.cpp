@@ -38,13 +38,15 @@ void check_hip(hipError_t err, const char* what) {
     TORCH_CHECK(err == hipSuccess, what, " failed: ", hipGetErrorString(err));
 }
 
+constexpr int64_t kMaxStride = 0x7fffffff;   // of the strided entries
+
 // x [B, T, H, 128] as the kernels read it in place: a head's elements and the
 // heads next to each other, 16-byte aligned rows; anything else is copied.
 at::Tensor head_rows(const at::Tensor& x) {
     const int64_t H = x.size(2), D = x.size(3);
     const bool ok = x.stride(3) == 1 && (H <= 1 || x.stride(2) == D) &&
-                    (x.size(0) <= 1 || (x.stride(0) % 8 == 0 && x.stride(0) <= 0x7fffffff)) &&
-                    (x.size(1) <= 1 || (x.stride(1) % 8 == 0 && x.stride(1) <= 0x7fffffff));
+                    (x.size(0) <= 1 || (x.stride(0) % 8 == 0 && x.stride(0) <= kMaxStride)) &&
+                    (x.size(1) <= 1 || (x.stride(1) % 8 == 0 && x.stride(1) <= kMaxStride));
     at::Tensor r = ok ? x : x.contiguous();
     return reinterpret_cast<uintptr_t>(r.data_ptr()) % 16 == 0 ? r : r.clone(at::MemoryFormat::Contiguous);
 }
@@ -308,7 +310,7 @@ at::Tensor recurrent_impl(const at::Tensor& q, const at::Tensor& k, const at::Te
     TORCH_CHECK(!state_in.defined() || state_in.is_contiguous(),
                 "state is updated in place and must be contiguous");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
-    const at::Tensor qc = head_rows(q), kc = head_rows(k), vc = head_rows(v);
+    at::Tensor qc = head_rows(q), kc = head_rows(k), vc = head_rows(v);
     auto gc = g.contiguous();
     auto bc = beta.contiguous();
     const int64_t B = qc.size(0), T = qc.size(1), HQK = qc.size(2), DK = qc.size(3);
@@ -329,6 +331,23 @@ at::Tensor recurrent_impl(const at::Tensor& q, const at::Tensor& k, const at::Te
             if (state_in.defined()) state_out.copy_(state_in);
             else state_out.zero_();
         }
+    }
+    if (B > 1 && std::max({qc.stride(0), kc.stride(0), vc.stride(0)}) > kMaxStride) {
+        // a packed tensor of 2^31 elements a batch: the entries for packed
+        // rows, which step the state in place
+        qc = qc.contiguous();
+        kc = kc.contiguous();
+        vc = vc.contiguous();
+        if (!state_out.is_same(state_in)) {
+            if (state_in.defined()) state_out.copy_(state_in);
+            else state_out.zero_();
+        }
+        auto step = qk_l2norm ? deltanet_recurrent_step_l2norm : deltanet_recurrent_step;
+        check_hip(step(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), gc.data_ptr<float>(),
+                       bc.data_ptr<float>(), o.data_ptr(), state_out.data_ptr<float>(), (int)B,
+                       (int)T, (int)HV, (int)HQK, (int)DK, (int)DV, current_stream()),
+                  "deltanet_recurrent_step");
+        return o;
     }
     const at::Tensor& from = T == 0 ? state_out : state_in;
     auto batch = [&](const at::Tensor& x) { return B > 1 ? x.stride(0) : 0; };

@@ -62,6 +62,7 @@ _PROTOS = {
                                        [hipStream_t]),
     "deltanet_recurrent_step_strided": (hipError_t, [vp, vp, vp, fp, fp, vp, fp, fp] +
                                         [c_int] * 4 + [c_int64] * 6 + [c_int, hipStream_t]),
+    "deltanet_recurrent_row_offset": (c_size_t, [c_int] * 5),
     "deltanet_chunk_prefill_strided": (hipError_t, [vp, c_int64, vp, c_int64, vp, c_int64, fp, fp,
                                                     vp, fp, fp, i32p] + [c_int] * 6 +
                                        [vp, c_size_t, hipStream_t]),

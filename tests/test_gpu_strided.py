@@ -64,3 +64,25 @@ def test_decode_new_state_without_tokens(ops, dev):
     assert o.shape == (2, 0, 4, 128) and torch.equal(s, s0) and s.data_ptr() != s0.data_ptr()
     with pytest.raises(RuntimeError):
         ops.recurrent_step_new(*[t[:0] for t in e], s0[:0])
+
+
+@pytest.mark.parametrize("norm", [False, True])
+def test_decode_batches_of_2_31_elements(ops, dev, norm):
+    """v's batches lie 2^31 elements apart (T HV = 2^24): the second batch as
+    it steps alone, in place and into a new state."""
+    B, T, HK, HV = 2, 1024, 1, 16384
+    print(f"[strided] decode B={B} T={T} HK={HK} HV={HV} norm={norm}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(21)
+    kw = dict(generator=gen, device=dev)
+    q, k = (torch.randn(B, T, HK, 128, **kw).mul_(0.1).bfloat16() for _ in range(2))
+    v = torch.randn(B, T, HV, 128, dtype=torch.bfloat16, **kw)
+    g = -torch.rand(B, T, HV, **kw)
+    beta = torch.rand(B, T, HV, **kw)
+    s0 = torch.randn(B, HV, 128, 128, **kw)
+    s1 = s0[1:].clone()
+    o1 = ops.recurrent_step(q[1:], k[1:], v[1:], g[1:], beta[1:], s1, qk_l2norm=norm)
+    o, s = ops.recurrent_step_new(q, k, v, g, beta, s0, qk_l2norm=norm)
+    assert torch.equal(o[1:], o1) and torch.equal(s[1:], s1)
+    del o, s
+    o = ops.recurrent_step(q, k, v, g, beta, s0, qk_l2norm=norm)
+    assert torch.equal(o[1:], o1) and torch.equal(s0[1:], s1)

@@ -33,3 +33,17 @@ def test_decode_strided_refuses(B, T, s_in, qb, v, vt):
     assert capi.lib().deltanet_recurrent_step_strided(
         P, P, v, P, P, P, s_in, P, B, T, 2, 2, qb, 256, 256, 256, 256, vt, 0,
         None) == capi.HIP_ERROR_INVALID_VALUE
+
+
+@pytest.mark.parametrize("T,heads,b,t,h", [
+    (1, 1, 0, 0, 0),
+    (3, 32, 5, 2, 31),
+    (524288, 32, 1, 0, 0),          # a batch of 2^31 elements
+    (524289, 32, 1, 524288, 31),
+    (1024, 16384, 1, 1023, 16383),
+    (4096, 8192, 200, 4095, 8191),
+])
+def test_decode_packed_rows_in_64_bits(T, heads, b, t, h):
+    """Batch strides of the packed decode entries, past 2^31 elements too."""
+    assert capi.lib().deltanet_recurrent_row_offset(T, heads, b, t, h) == \
+        ((b * T + t) * heads + h) * 128
