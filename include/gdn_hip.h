@@ -220,9 +220,9 @@ hipError_t deltanet_recurrent_step_l2norm(const void* q, const void* k, const vo
 /* deltanet_recurrent_step (qk_l2norm != 0: _l2norm) for q, k, v rows that lie
  * apart, and for a state that goes to another buffer: heads lie next to each
  * other (128 elements), batches and tokens q_batch, q_token, .. elements
- * apart (below 2^31); v 8-byte aligned, its strides multiples of 4.  state_in NULL: zeros;
- * state_in may be state_out.  Head dims 128.  T = 0 needs state_in =
- * state_out (nothing is done). */
+ * apart (below 2^31); v 8-byte aligned, its strides multiples of 4; the states
+ * aligned as floats.  state_in NULL: zeros; state_in may be state_out.  Head
+ * dims 128.  T = 0 needs state_in = state_out (nothing is done). */
 hipError_t deltanet_recurrent_step_strided(const void* q, const void* k, const void* v,
                                            const float* g, const float* beta, void* o,
                                            const float* state_in, float* state_out, int B, int T,

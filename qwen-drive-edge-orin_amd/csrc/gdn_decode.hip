@@ -49,7 +49,9 @@ static_assert(kRowGroups * kRowsPerThread == kDK && kRowGroups % 4 == 0, "row gr
 // caller that keeps the old state needs no copy of it, one pass over the
 // state instead of two (a B=24 HV=32 layer step with conv and norm: 49.5 ->
 // 26 us).  Reading and writing one buffer is safe: a thread reads its
-// elements before it writes them, and no other thread touches them.
+// elements before it writes them, and no other thread touches them.  The
+// state is the caller's and may be a view at any float (f32x4_a4; the hardware
+// takes 16-byte accesses at 4-byte addresses).
 struct DecStrides {   // elements; a batch's T tokens may span more than 31 bits
     int64_t qb, kb, vb;
     int qt, kt, vt;
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(kDecThreads) void gdn_recurrent_kernel(
 #pragma unroll
         for (int m = 0; m < kRowsPerThread; ++m)
             s[m] = __builtin_nontemporal_load(
-                reinterpret_cast<const f32x4*>(S + (rg + kRowGroups * m) * kDV + c0) + cb);
+                reinterpret_cast<const f32x4_a4*>(S + (rg + kRowGroups * m) * kDV + c0) + cb);
     } else {
 #pragma unroll
         for (int m = 0; m < kRowsPerThread; ++m) s[m] = zero4();
@@ -195,7 +197,8 @@ __global__ __launch_bounds__(kDecThreads) void gdn_recurrent_kernel(
     float* S = state_out + sb;
 #pragma unroll
     for (int m = 0; m < kRowsPerThread; ++m)
-        __builtin_nontemporal_store(s[m], reinterpret_cast<f32x4*>(S + (rg + kRowGroups * m) * kDV + c0) + cb);
+        __builtin_nontemporal_store(
+            s[m], reinterpret_cast<f32x4_a4*>(S + (rg + kRowGroups * m) * kDV + c0) + cb);
 }
 
 }  // namespace

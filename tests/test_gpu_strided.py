@@ -66,6 +66,20 @@ def test_decode_new_state_without_tokens(ops, dev):
         ops.recurrent_step_new(*[t[:0] for t in e], s0[:0])
 
 
+def test_decode_state_at_any_float(ops, dev):
+    """The state a contiguous view that starts one float into its buffer."""
+    q, k, v, g, beta, s0 = [t.to(dev) for t in gc.make_gdn_inputs(9, B=2, T=2, HK=2, HV=4)]
+    s_ref = s0.clone()
+    o_ref = ops.recurrent_step(q, k, v, g, beta, s_ref)
+    for off in (1, 2, 3):
+        s = torch.cat([s0.flatten()[:off], s0.flatten()])[off:].view(s0.shape)
+        assert s.data_ptr() % 16 == 4 * off
+        o, s_new = ops.recurrent_step_new(q, k, v, g, beta, s)
+        assert torch.equal(o, o_ref) and torch.equal(s_new, s_ref) and torch.equal(s, s0)
+        o = ops.recurrent_step(q, k, v, g, beta, s)
+        assert torch.equal(o, o_ref) and torch.equal(s, s_ref)
+
+
 @pytest.mark.parametrize("norm", [False, True])
 def test_decode_batches_of_2_31_elements(ops, dev, norm):
     """v's batches lie 2^31 elements apart (T HV = 2^24): the second batch as
