@@ -27,6 +27,7 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef f32x4 f32x4_a4 __attribute__((aligned(4)));   // in memory, wherever a float may lie
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));   // in memory at an 8-byte address
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kDK = 128;     // key head dim (only validated size)

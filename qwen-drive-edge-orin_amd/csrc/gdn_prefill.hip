@@ -2533,7 +2533,8 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
     // again: non-temporal (2 x 3200 tokens HV32 HK32 153.2 -> 148.1 us, 4 x
     // 1141 HV32 75.0 -> 70.9).  The reads and their wait are one asm
     // block: the compiler would place a wait for every direct-to-LDS load in
-    // front of an LDS read of its own.
+    // front of an LDS read of its own.  o's base needs the 8-byte alignment of
+    // the narrower instances' stores, no more.
     auto store_o = [&](int c) {
         const int rows = min(kChunk, x.len - c * kChunk);
         u32x4 v0, v1;
@@ -2550,7 +2551,7 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
             if (r < rows)
                 __builtin_nontemporal_store(
                     i ? v1 : v0,
-                    reinterpret_cast<u32x4*>(
+                    reinterpret_cast<u32x4_a8*>(
                         a.o + ((size_t)(x.tok_base + c * kChunk + r) * a.HV + x.hv) * kDV +
                         kWideCols * x.sl + 8 * p));
         }

@@ -15,7 +15,7 @@ from gdn_hip import capi
 pytestmark = pytest.mark.gpu
 
 
-def _run(dev, d, cu, cols):
+def _run(dev, d, cu, cols, o_offset=0):
     lib = capi.lib()
     q, k, v, g, beta, s0 = d
     B, T, HK, D = q.shape
@@ -25,7 +25,8 @@ def _run(dev, d, cu, cols):
             else lib.deltanet_prefill_live_workspace_size)
     wsb = size(T, N, HV, D, D, 64) if cu is not None else size(B, T, HV, D, D, 64)
     ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
-    o = torch.zeros_like(v)
+    o = torch.zeros(v.numel() + 8, dtype=v.dtype, device=dev)
+    o = o[o_offset:o_offset + v.numel()].view(v.shape)
     sf = torch.zeros(N, HV, D, D, device=dev)
     cud = cu.to(dev) if cu is not None else None
     print(f"[wide] cols={cols} N={N} T={T} HK={HK} HV={HV}", flush=True)
@@ -61,3 +62,12 @@ def test_wide_equals_16col_batch(dev, B, T, HK, HV):
         o16, s16 = _run(dev, d[:5] + [s0], None, 16)
         o, s = _run(dev, d[:5] + [s0], None, 128)
         assert torch.equal(o, o16) and torch.equal(s, s16)
+
+
+def test_wide_o_at_an_8_byte_address(dev):
+    """o's rows 8 bytes past a 16-byte boundary, all the narrower instances ask for."""
+    d = [t.to(dev) for t in gc.make_gdn_inputs(23, B=2, T=130, HK=2, HV=4, g_shift=2.0)]
+    o16, s16 = _run(dev, d, None, 16, o_offset=4)
+    o, s = _run(dev, d, None, 128, o_offset=4)
+    assert o.data_ptr() % 16 == 8
+    assert torch.equal(o, o16) and torch.equal(s, s16)
