@@ -48,7 +48,9 @@ hipError_t deltanet_chunk_prefill_kernel(const void* q, const void* k, const voi
  * scan's bounded waits limited to spin_limit polls each (the library's own
  * limit is 2^20).  With a small limit the waits give up, every kernel still
  * returns normally, and deltanet_prefill_status then reports
- * hipErrorLaunchTimeOut: the test of that error path. */
+ * hipErrorLaunchTimeOut: the test of that error path.  The wide scan instance,
+ * which waits for no stage, is never taken under a limit other than the
+ * library's. */
 hipError_t deltanet_chunk_prefill_spin(const void* q, const void* k, const void* v,
                                        const float* g, const float* beta, void* o,
                                        const float* initial_state, float* final_state, int B,
@@ -73,6 +75,13 @@ hipError_t deltanet_chunk_prefill_cols(const void* q, const void* k, const void*
                                        const int32_t* cu_seqlens, int num_seqs, int T, int HV,
                                        int HQK, void* workspace, size_t workspace_bytes,
                                        hipStream_t stream, int slice_cols, unsigned spin_limit);
+
+/* The scan instance that the library chooses by itself (host only): value
+ * columns per work-group, 16, 32 or 64, for `chunks` chunks in all over
+ * num_seqs sequences on a device of `cus` CUs, spin_limit as in
+ * deltanet_chunk_prefill_cols; -1 for invalid arguments. */
+int deltanet_prefill_scan_cols(size_t chunks, int num_seqs, int HV, int HQK, int cus,
+                               unsigned spin_limit);
 
 /* Host mirror of the kernels' sequence bookkeeping for a packed batch
  * (host memory, no GPU involved): for each sequence s its first chunk id,

@@ -2867,23 +2867,28 @@ int device_cus() {
     return n;
 }
 
+// Bytes of records that the prep writes for nch chunks.
+size_t record_bytes(size_t nch, int HV, int HK) {
+    return nch * HV * (3 * kTriBytes + kWBytes + kGateBytes) + nch * HK * (kQBytes + kKTBytes);
+}
+
 // Scan instance (value columns per work-group): 16-column groups while they
 // fit on the CUs at once (one group per CU), the paired 32-column groups once
 // they would run in rounds (then the halves' shared operands halve the
 // rounds), the wide 64-column groups once the paired ones would (paired and
 // wide, 3 x 1141 tokens HV32: 74.7 and 59.8 us; 6 x 256: 43.9 and 35.2; 8
 // packed prompts, 19,861 tokens: 430 and 340), or, with more than 48 heads,
-// where each group's operands come from beyond its L2 (`far`: every head has
-// its own Q and K^T, or the records outgrow the memory-side cache) and the
-// wide groups' half as many fetches count (2 x 2000 tokens HV32 HK32: 94.7
-// and 86.6; 2 x 4096 HV32 HK16: 171 and 166; but 2 x 1141 HV32 HK16 45.5 and
-// 49, and 48 heads 117.5 and 118.7).  cols forces one (diagnostics); the debug
-// dump and the norm epilogue exist in the 16-column instance only.
-int scan_cols(int cols, int N, int HV, int dump_debug, bool norm, bool far) {
-    if (cols) return cols;
-    if (dump_debug || norm) return kSliceCols;
-    const long long heads = (long long)N * HV, cus = device_cus();
+// where each group's operands come from beyond its L2 (every head has its own
+// Q and K^T, or the records outgrow the memory-side cache) and the wide
+// groups' half as many fetches count (2 x 2000 tokens HV32 HK32: 94.7 and
+// 86.6; 2 x 4096 HV32 HK16: 171 and 166; but 2 x 1141 HV32 HK16 45.5 and 49,
+// and 48 heads 117.5 and 118.7).  A caller's own spin limit keeps to the
+// instances that have bounded waits.
+int scan_cols(size_t nch, int N, int HV, int HK, long long cus, unsigned spin) {
+    const long long heads = (long long)N * HV;
     if (heads * kSlicesPerHead <= cus) return kSliceCols;
+    if (spin != kDefaultSpin) return kPairCols;
+    const bool far = record_bytes(nch, HV, HK) > kNtRecordBytes || HV == HK;
     if (far && heads * 16 > cus * 3) return kWideCols;
     return heads * kPairsPerHead <= cus ? kPairCols : kWideCols;
 }
@@ -2895,10 +2900,12 @@ hipError_t launch_prefill(PrepIn in, int raw, void* o, const float* s0, float* s
                           int only = -1, unsigned spin = kDefaultSpin,
                           const NormIn* norm = nullptr, int cols = 0) {
     // records written non-temporally: see st_through
-    const size_t written = nch_bound * HV * (3 * kTriBytes + kWBytes + kGateBytes) +
-                           nch_bound * HK * (kQBytes + kKTBytes);
-    const bool nt = !dump_debug && written > kNtRecordBytes;
-    const int width = scan_cols(cols, N, HV, dump_debug, norm != nullptr, nt || HV == HK);
+    const bool nt = !dump_debug && record_bytes(nch_bound, HV, HK) > kNtRecordBytes;
+    // cols forces a scan instance (diagnostics); the debug dump and the norm
+    // epilogue exist in the 16-column one only
+    const int width = cols                ? cols
+                      : dump_debug || norm ? kSliceCols
+                                           : scan_cols(nch_bound, N, HV, HK, device_cus(), spin);
     if (width != kSliceCols && (dump_debug || norm)) return hipErrorInvalidValue;
     if (in.qts < 0) in.qts = HK * kDK;
     if (in.kts < 0) in.kts = HK * kDK;
@@ -3097,10 +3104,10 @@ extern "C" hipError_t deltanet_chunk_prefill_norm_fused(
     // The epilogue lives in the 16-column scan; where the plain prefill would
     // take the paired 32-column instance (more slice groups than CUs) the
     // two-kernel path runs instead.
-    if (scan_cols(0, B, HV, 0, false, false) != kSliceCols)
+    const size_t nc = (size_t)B * ((T + kChunk - 1) / kChunk);
+    if (scan_cols(nc, B, HV, HQK, device_cus(), kDefaultSpin) != kSliceCols)
         return prefill_then_norm(q, k, v, g, beta, z, norm_weight, eps, y, initial_state,
                                  final_state, B, T, HV, HQK, workspace, workspace_bytes, stream);
-    const size_t nc = (size_t)B * ((T + kChunk - 1) / kChunk);
     const NormIn n{static_cast<const uint16_t*>(z), static_cast<const uint16_t*>(norm_weight), eps};
     return launch_prefill(plain_in(q, k, v, g, beta), 0, y, initial_state, final_state, nullptr,
                           B, T, B * T, HV, HQK, nc, workspace, workspace_bytes, stream, 0, nullptr,
@@ -3158,6 +3165,12 @@ extern "C" hipError_t deltanet_chunk_prefill_cols(const void* q, const void* k, 
     return launch_prefill(plain_in(q, k, v, g, beta), 0, o, initial_state, final_state, nullptr,
                           num_seqs, T, num_seqs * T, HV, HQK, nc, workspace, workspace_bytes,
                           stream, 0, nullptr, -1, spin, nullptr, slice_cols);
+}
+
+extern "C" int deltanet_prefill_scan_cols(size_t chunks, int num_seqs, int HV, int HQK, int cus,
+                                          unsigned spin_limit) {
+    if (num_seqs <= 0 || !dims_ok(HV, HQK, kDK, kDV, kChunk) || cus <= 0) return -1;
+    return scan_cols(chunks, num_seqs, HV, HQK, cus, spin_limit ? spin_limit : kDefaultSpin);
 }
 
 extern "C" int deltanet_prefill_kernel_count(void) { return kPrefillKernels; }

@@ -48,6 +48,7 @@ _PROTOS = {
                                     [vp, c_size_t, hipStream_t, ct.c_uint]),
     "deltanet_chunk_prefill_cols": (hipError_t, [vp, vp, vp, fp, fp, vp, fp, fp, vp] + [c_int] * 4 +
                                     [vp, c_size_t, hipStream_t, c_int, ct.c_uint]),
+    "deltanet_prefill_scan_cols": (c_int, [c_size_t] + [c_int] * 4 + [ct.c_uint]),
     "deltanet_varlen_chunk_map": (c_int, [vp, c_int, c_int, vp, vp, vp, vp]),
     "deltanet_varlen_chunks_before": (c_int, [vp, c_int, c_int, c_int, c_int]),
     "deltanet_prefill_twolevel_workspace_size": (c_size_t, [vp, c_int, c_int, c_int, c_int]),

@@ -71,3 +71,20 @@ def test_wide_o_at_an_8_byte_address(dev):
     o, s = _run(dev, d, None, 128, o_offset=4)
     assert o.data_ptr() % 16 == 8
     assert torch.equal(o, o16) and torch.equal(s, s16)
+
+
+def test_spin_limit_keeps_bounded_waits(dev):
+    """Heads for which the library takes the wide instance: a caller's spin
+    limit is met by one with bounded waits, and reported."""
+    lib = capi.lib()
+    d = [t.to(dev) for t in gc.make_gdn_inputs(29, B=5, T=200, HK=8, HV=16, g_shift=2.0)]
+    o, sf = torch.empty_like(d[2]), torch.empty_like(d[5])
+    wsb = lib.deltanet_prefill_live_workspace_size(5, 200, 16, 128, 128, 64)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    for spin, want in ((0, capi.HIP_ERROR_LAUNCH_TIMEOUT), (1 << 20, capi.HIP_SUCCESS)):
+        print(f"[wide] spin={spin} N=5 T=200 HK=8 HV=16", flush=True)
+        assert lib.deltanet_chunk_prefill_spin(
+            *[capi.ptr(t) for t in d[:5]], o.data_ptr(), d[5].data_ptr(), sf.data_ptr(), 5, 200, 16,
+            8, ws.data_ptr(), wsb, stream, ct.c_uint(spin)) == capi.HIP_SUCCESS
+        assert lib.deltanet_prefill_status(ws.data_ptr(), wsb, stream) == want
