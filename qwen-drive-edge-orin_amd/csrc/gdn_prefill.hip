@@ -385,6 +385,14 @@ __device__ bool locate_chunk(const int32_t* cu, int N, int T, int total, int cid
 // asm statement, so the 16-byte form carries its own s_nop.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr size_t kNtRecordBytes = size_t(192) << 20;
+// Where records just below that are written through, the prep takes its last
+// chunk first: the scan starts at the first chunks, whose records are then the
+// newest in the memory-side cache (7600 tokens HV32, 190 MB: 198 -> 191 us; 2 x
+// 3600, 182 MB: 152.8 -> 150.1; 172-175 MB within 1 % either way).  With fewer
+// records the first chunk first is the better order (T3200, 80 MB: 84.4 against
+// 85.4; T77 14.38 against 14.45), non-temporally written ones do not care.  The
+// order is an instance of its own: chosen at run time it cost T77 0.05 us.
+constexpr size_t kLastFirstBytes = size_t(176) << 20;
 template <bool kNt = false, typename V>
 __device__ __forceinline__ void st_through(V* p, const V& v) {
     static_assert(sizeof(V) == 4 || sizeof(V) == 8 || sizeof(V) == 16, "4, 8 or 16 bytes");
@@ -489,7 +497,7 @@ __device__ inline void am_products(const half8 (&ka)[4][4], const half8 (&qf)[4]
     }
 }
 
-template <bool kDbg, int kRaw, bool kNt = false, bool kStrided = false>
+template <bool kDbg, int kRaw, bool kNt = false, bool kStrided = false, bool kLastFirst = false>
 __global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(
     PrepIn in, const int32_t* __restrict__ cu, int N, int T, int total, int HV, int HK,
     int nch_bound, float scale, Workspace ws) {
@@ -516,8 +524,9 @@ __global__ __launch_bounds__(kPrepThreads, 4) void gdn_prep_kernel(
     const int L = blockIdx.x;
     const int rest = L >> 3;
     const int z = (rest / rep) * 8 + (L & 7);
-    const int cid = z / HK, hk = z - cid * HK;
-    if (cid >= nch_bound) return;
+    const int cz = z / HK, hk = z - cz * HK;
+    if (cz >= nch_bound) return;
+    const int cid = kLastFirst ? nch_bound - 1 - cz : cz;   // kLastFirstBytes
     const int member = rest % rep;
     const int hv = hk * rep + member;
 
@@ -2902,12 +2911,18 @@ int scan_cols(size_t nch, int N, int HV, int HK, long long cus, unsigned spin) {
 }
 
 // The prep and scan instances for rows packed or apart (kStrided)
+template <int kRaw, bool kStrided>
+auto prep_order(bool nt, bool last_first) {
+    return nt           ? gdn_prep_kernel<false, kRaw, true, kStrided>
+           : last_first ? gdn_prep_kernel<false, kRaw, false, kStrided, true>
+                        : gdn_prep_kernel<false, kRaw, false, kStrided>;
+}
+
 template <bool kStrided>
-auto prep_kernel(int raw, bool nt) {
+auto prep_kernel(int raw, bool nt, bool last_first) {
     if constexpr (!kStrided)
-        if (raw == 2) return nt ? gdn_prep_kernel<false, 2, true> : gdn_prep_kernel<false, 2>;
-    return raw ? (nt ? gdn_prep_kernel<false, 1, true, kStrided> : gdn_prep_kernel<false, 1, false, kStrided>)
-               : (nt ? gdn_prep_kernel<false, 0, true, kStrided> : gdn_prep_kernel<false, 0, false, kStrided>);
+        if (raw == 2) return prep_order<2, false>(nt, last_first);
+    return raw ? prep_order<1, kStrided>(nt, last_first) : prep_order<0, kStrided>(nt, last_first);
 }
 
 template <bool kStrided>
@@ -2931,7 +2946,8 @@ hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, f
                           int only = -1, unsigned spin = kDefaultSpin,
                           const NormIn* norm = nullptr, int cols = 0) {
     // records written non-temporally: see st_through
-    const bool nt = !dump_debug && record_bytes(nch_bound, HV, HK) > kNtRecordBytes;
+    const size_t records = record_bytes(nch_bound, HV, HK);
+    const bool nt = !dump_debug && records > kNtRecordBytes;
     // cols forces a scan instance (diagnostics); the debug dump and the norm
     // epilogue exist in the 16-column one only
     const int width = cols                ? cols
@@ -2971,9 +2987,10 @@ hipError_t launch_prefill(const PrepIn& in, int raw, void* o, const float* s0, f
         const int rep = HV / HK;
         const size_t groups = (nch_bound * (size_t)HK + 7) / 8;
         const size_t grid = std::max<size_t>(groups * 8 * rep, 1);
-        auto kern = strided ? prep_kernel<true>(raw, nt)
+        const bool last_first = records > kLastFirstBytes;   // written through
+        auto kern = strided ? prep_kernel<true>(raw, nt, last_first)
                     : dump_debug ? gdn_prep_kernel<true, 0>
-                                 : prep_kernel<false>(raw, nt);
+                                 : prep_kernel<false>(raw, nt, last_first);
         PrepIn pin = in;
         pin.s0 = s0;
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kPrepThreads), 0, stream, pin, cu, N, T,
