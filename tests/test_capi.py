@@ -269,7 +269,7 @@ def test_twolevel_rejects_on_host(lib):
 
 
 def test_cols_entry_rejects_on_host(lib):
-    """deltanet_chunk_prefill_cols: a slice width other than 0, 16 or 32, bad
+    """deltanet_chunk_prefill_cols: a slice width other than 0, 16, 32 or 128, bad
     head counts, no sequences, a short workspace and missing pointers are
     rejected before any launch."""
     d = 16

@@ -75,6 +75,21 @@ def test_rejects_host_tensors():
         m.recurrent_gated_delta_rule(q, q, v, g, g)
 
 
+def test_native_decode_call_leaves_other_arguments():
+    """What is not the ordinary decode call is None there, never an error."""
+    import torch
+
+    native = _adapter().gdn_hip.load()._recurrent_ordinary
+    q = torch.zeros(1, 1, 2, 128, dtype=torch.bfloat16)
+    g = torch.zeros(1, 1, 2)
+    s = torch.zeros(1, 2, 128, 128)
+    assert native(q, q, q, g, g, s, True) is None          # host tensors
+    assert native(q, q, q, g, g, None, False) is None
+    assert native(None, q, q, g, g, s, True) is None
+    assert native(q, q, q, 0.5, g, s, True) is None
+    assert native(q, q, q, g, g, 0, True) is None
+
+
 @pytest.mark.parametrize("env,expect", [(None, False), ("0", False), ("1", True)])
 def test_checked_mode_reaches_the_op(monkeypatch, env, expect):
     """GDN_HIP_CHECKED=1 at import makes every prefill call ask the op to check

@@ -80,12 +80,13 @@ def _check(o, o_ref, s, s_ref, tag):
 
 
 @pytest.mark.parametrize("B,T,HK,HV", [(1, 150, 2, 4), (2, 64, 1, 2), (1, 1141, 2, 4),
-                                       (1, 1141, 16, 32), (2, 300, 16, 32)])
+                                       (1, 1141, 16, 32), (3, 130, 8, 16), (2, 300, 16, 32)])
 def test_chunk_matches_transformers(fla_ops, torch_ref, dev, B, T, HK, HV):
     """(1, 1141, 16, 32) is the planner's layer: 16 k-heads expanded to the 32
     v-heads before the call (modeling_qwen3_5.py:500-502), as transformers
-    hands them to fla.  (2, 300, 16, 32) has more (sequence, head) pairs than
-    one 16-column scan group per CU covers, so it runs the paired scan's
+    hands them to fla.  (3, 130, 8, 16) and (2, 300, 16, 32) have more
+    (sequence, head) pairs than one 16-column scan group per CU covers: they
+    run the paired and, with a k-head for each of 64 v-heads, the wide scan's
     raw-bf16 instance."""
     q, k, v, g, beta, s0 = _layer_inputs(B, T, HK, HV, seed=T + HV)
     o_ref, s_ref = torch_ref[0](q.float(), k.float(), v.float(), g, beta, initial_state=s0,
@@ -168,3 +169,39 @@ def test_scale_and_shape_checks(fla_ops, torch_ref, dev):
     with pytest.raises(NotImplementedError):
         fla_ops.chunk_gated_delta_rule(*[t[..., :64].contiguous().to(dev) if t.dim() == 4 else t.to(dev)
                                          for t in (q, k, v, g, beta)])
+
+
+def test_recurrent_other_forms_than_the_ordinary(fla_ops, dev):
+    """Mixed dtypes, a strided state, a state that requires a gradient and an
+    explicit default scale leave the native call for the general path: the
+    ordinary call's values, and autograd sees a copy of the state."""
+    q, k, v, g, beta, s0 = [t.to(dev) for t in _layer_inputs(2, 1, 2, 4, seed=31)]
+    beta = beta.float()
+    kw = dict(output_final_state=True, use_qk_l2norm_in_kernel=True)
+    o_ref, s_ref = fla_ops.recurrent_gated_delta_rule(q, k, v, g, beta, initial_state=s0, **kw)
+    native = fla_ops.gdn_hip.load()._recurrent_ordinary
+    assert native(q, k, v, g, beta, s0, True) is not None
+
+    def same(o, s):
+        assert torch.equal(o, o_ref) and torch.equal(s.detach(), s_ref)
+
+    b16 = beta.bfloat16()
+    assert native(q, k, v, g, b16, s0, True) is None
+    o, s = fla_ops.recurrent_gated_delta_rule(q, k, v, g, b16, initial_state=s0, **kw)
+    o2, s2 = fla_ops.recurrent_gated_delta_rule(q, k, v, g, b16.float(), initial_state=s0, **kw)
+    assert torch.equal(o, o2) and torch.equal(s, s2)
+    st = s0.transpose(2, 3).contiguous().transpose(2, 3)
+    assert native(q, k, v, g, beta, st, True) is None
+    same(*fla_ops.recurrent_gated_delta_rule(q, k, v, g, beta, initial_state=st, **kw))
+    same(*fla_ops.recurrent_gated_delta_rule(q, k, v, g, beta, scale=128 ** -0.5, initial_state=s0,
+                                             **kw))
+    leaf = s0.clone().requires_grad_()
+    assert native(q, k, v, g, beta, leaf, True) is None
+    o, s = fla_ops.recurrent_gated_delta_rule(q, k, v, g, beta, initial_state=leaf, **kw)
+    same(o, s)
+    assert s.requires_grad and torch.equal(leaf.detach(), s0)
+    with torch.no_grad():
+        assert native(q, k, v, g, beta, leaf, True) is not None
+    assert native(q, k, v[:, :, :3], g, beta, s0, True) is None
+    with pytest.raises(ValueError):
+        fla_ops.recurrent_gated_delta_rule(q, k, v[:, :, :3], g, beta, initial_state=s0, **kw)

@@ -50,6 +50,12 @@ def test_fused_batch_gqa(ops, dev):
     _fused(ops, dev, *gc.fused_inputs(24, B=2, T=200, HK=16, HV=32), tag="fp16 B2 T200 HV32")
 
 
+def test_fused_bf16_paired_scan(ops, dev):
+    """B=2 HV=32 in bf16: the paired scan's raw-bf16 instance."""
+    _fused(ops, dev, *gc.fused_inputs(25, B=2, T=200, HK=16, HV=32, dtype=torch.bfloat16),
+           tag="bf16 B2 T200 HV32")
+
+
 def test_fused_empty_sequence_keeps_state(ops, dev):
     q, k, v, a, b, A_log, dt_bias, s0 = gc.fused_inputs(22, B=1, T=0, HK=2, HV=4)
     st = s0.to(dev).contiguous()

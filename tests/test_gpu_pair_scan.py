@@ -2,11 +2,11 @@
 (sequence, head)) against the 16-column instance, through the C ABI's
 deltanet_chunk_prefill_cols: bitwise the same o and final state, since each
 half runs the 16-column arithmetic operation for operation.  The library picks
-the paired instance by itself once the 16-column groups outnumber the CUs, so
-the oracle-parity tests of packed batches (test_gpu_prefill.py: the
-8-sequence batch, the edge lengths, the per-sequence equality) and of the fp16
-batch (test_gpu_fused.py: B=2 HV=32) run it too; here both instances are
-forced on the same inputs, including shapes where the library would not pick
+the paired instance by itself once the 16-column groups outnumber the CUs and
+while its own do not (33 to 64 heads on 256 CUs; the wide one beyond, and from
+49 on where operands come from far), so the oracle-parity tests of the fused
+batches (test_gpu_fused.py: B=2 HV=32 in fp16 and bf16) run it too; here both
+instances are forced on the same inputs, including shapes where the library would not pick
 the paired one, and the paired instance's bounded waits are checked to give up
 cleanly.
 """

@@ -148,9 +148,9 @@ def test_long_sequences(ops, dev, B, T, HK, HV, g_shift):
 
 
 def test_workspace_beyond_the_memory_side_cache(ops, dev):
-    """B2 T4096 HV32 HK16: 276 MB of workspace, more than the 256 MB
-    memory-side cache, so the prep writes its records non-temporally; 512
-    16-column groups, so the paired scan runs."""
+    """B2 T4096 HV32 HK16: 276 MB of workspace and 204 MB of records, more
+    than the memory-side cache keeps beside the inputs, so the prep writes
+    them non-temporally; 64 heads with such records, so the wide scan runs."""
     q, k, v, g, beta, s0 = gc.make_gdn_inputs(4096, B=2, T=4096, HK=16, HV=32, g_shift=2.0)
     _run_and_check(ops, dev, q, k, v, g, beta, s0, tag="T4096 B2 HV32 (276 MB workspace)")
 

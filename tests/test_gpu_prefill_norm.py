@@ -55,7 +55,7 @@ def test_prefill_norm_default_is_two_steps(ops, dev):
                                        (8, 70, 32, 64)])
 def test_prefill_norm_fused_matches_two_steps(ops, dev, B, T, HK, HV):
     """(8, 70, 32, 64) has 4096 slice groups, more than the chip's CUs: the
-    fused entry then takes the two-kernel path (with the paired scan), which
+    fused entry then takes the two-kernel path (with the wide scan), which
     must give the same bits."""
     q, k, v, g, beta, s0 = gc.make_gdn_inputs(31, B, T, HK, HV, g_shift=2.0)
     z, w = _z_w(32, v.shape)

@@ -35,6 +35,49 @@ def test_prefill_strided(ops, dev, form, B, T, HK, HV):
         assert o.is_contiguous() and torch.equal(o, o_ref) and torch.equal(s, s_ref)
 
 
+@pytest.mark.parametrize("form", ["slice", "odd_stride"])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("B,T,HK,HV", [(2, 130, 16, 32), (3, 70, 16, 16), (3, 70, 16, 32),
+                                       (2, 129, 32, 32)])
+def test_prefill_strided_paired_and_wide(ops, dev, form, norm, B, T, HK, HV):
+    """More (sequence, head) pairs than 16-column groups fit: the first two
+    run the paired scan, the others the wide one, against each sequence alone
+    and packed (the 16-column scan).  "slice" is read in place, "odd_stride"
+    copied."""
+    q, k, v, g, beta, s0 = [t.to(dev) for t in gc.make_gdn_inputs(11, B=B, T=T, HK=HK, HV=HV,
+                                                                  g_shift=2.0)]
+    f = FORMS[form]
+    print(f"[strided] prefill {form} B={B} T={T} HK={HK} HV={HV} norm={norm}", flush=True)
+    o, s = ops.chunk_prefill(f(q), f(k), f(v), g, beta, s0, qk_l2norm=norm)
+    for b in range(B):
+        i = slice(b, b + 1)
+        o1, s1 = ops.chunk_prefill(q[i], k[i], v[i], g[i], beta[i], s0[i], qk_l2norm=norm)
+        assert torch.equal(o[i], o1) and torch.equal(s[i], s1)
+
+
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("lens,HK,HV", [([70, 0, 1], 2, 4), ([65, 130], 16, 32),
+                                        ([0, 64, 63, 1, 200, 0], 8, 16)])
+def test_prefill_strided_packed_sequences(ops, dev, norm, lens, HK, HV):
+    """Ragged and empty sequences in rows of one buffer (16-column, paired and
+    wide scan) against the same rows without gaps, a sequence at a time."""
+    T = sum(lens)
+    q, k, v, g, beta, _ = [t.to(dev) for t in gc.make_gdn_inputs(12, B=1, T=T, HK=HK, HV=HV,
+                                                                 g_shift=2.0)]
+    s0 = 0.02 * torch.randn(len(lens), HV, 128, 128, generator=torch.Generator().manual_seed(6))
+    s0 = s0.to(dev)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    f = FORMS["slice"]
+    print(f"[strided] packed sequences {lens} HK={HK} HV={HV} norm={norm}", flush=True)
+    o, s = ops.chunk_prefill(f(q), f(k), f(v), g, beta, s0, cu_seqlens=cu.to(dev),
+                             qk_l2norm=norm)
+    for i in range(len(lens)):
+        t = slice(int(cu[i]), int(cu[i + 1]))
+        o1, s1 = ops.chunk_prefill(q[:, t], k[:, t], v[:, t], g[:, t], beta[:, t], s0[i:i + 1],
+                                   qk_l2norm=norm)
+        assert torch.equal(o[:, t], o1) and torch.equal(s[i:i + 1], s1)
+
+
 @pytest.mark.parametrize("form", sorted(FORMS))
 @pytest.mark.parametrize("B,T,HK,HV", [(1, 1, 2, 4), (3, 1, 2, 4), (2, 3, 1, 2)])
 def test_decode_strided_and_new_state(ops, dev, form, B, T, HK, HV):

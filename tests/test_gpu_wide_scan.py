@@ -88,3 +88,44 @@ def test_spin_limit_keeps_bounded_waits(dev):
             *[capi.ptr(t) for t in d[:5]], o.data_ptr(), d[5].data_ptr(), sf.data_ptr(), 5, 200, 16,
             8, ws.data_ptr(), wsb, stream, ct.c_uint(spin)) == capi.HIP_SUCCESS
         assert lib.deltanet_prefill_status(ws.data_ptr(), wsb, stream) == want
+
+
+@pytest.mark.parametrize("B,T,HK,HV", [(3, 193, 16, 32), (2, 65, 32, 32), (9, 128, 4, 8)])
+def test_wide_raw_rows_as_alone(ops, dev, B, T, HK, HV):
+    """Raw q and k (normalised in the kernels) and the fused step's raw bf16
+    and fp16 rows: each sequence as alone, where the 16-column scan runs."""
+    assert capi.lib().deltanet_prefill_scan_cols(B * ((T + 63) // 64), B, HV, HK, 256, 0) == 64
+    one = [slice(b, b + 1) for b in range(B)]
+    print(f"[wide] raw rows B={B} T={T} HK={HK} HV={HV}", flush=True)
+    d = [t.to(dev) for t in gc.make_gdn_inputs(83, B=B, T=T, HK=HK, HV=HV, g_shift=2.0)]
+    o, s = ops.chunk_prefill(*d, qk_l2norm=True)
+    for i in one:
+        o1, s1 = ops.chunk_prefill(*[t[i] for t in d], qk_l2norm=True)
+        assert torch.equal(o[i], o1) and torch.equal(s[i], s1)
+    for dtype in (torch.bfloat16, torch.float16):
+        q, k, v, a, b, A_log, dt_bias, s0 = [
+            t.to(dev) for t in gc.fused_inputs(84, B=B, T=T, HK=HK, HV=HV, dtype=dtype)]
+        s = s0.clone()
+        o = ops.chunk_prefill_fused(q, k, v, a, b, A_log, dt_bias, s)
+        for i in one:
+            s1 = s0[i].clone()
+            o1 = ops.chunk_prefill_fused(q[i], k[i], v[i], a[i], b[i], A_log, dt_bias, s1)
+            assert torch.equal(o[i], o1) and torch.equal(s[i], s1)
+
+
+def test_wide_noalloc_as_alone(ops, dev):
+    """The allocation-free entry on the wide scan (3 x 200 tokens, 32 heads:
+    384 chunk-heads, inside its array), each sequence as alone."""
+    lib = capi.lib()
+    B, T, HK, HV = 3, 200, 16, 32
+    d = [t.to(dev) for t in gc.make_gdn_inputs(85, B=B, T=T, HK=HK, HV=HV, g_shift=2.0)]
+    o, sf = torch.empty_like(d[2]), torch.empty_like(d[5])
+    stream = torch.cuda.current_stream().cuda_stream
+    print(f"[wide] noalloc B={B} T={T} HK={HK} HV={HV}", flush=True)
+    assert lib.deltanet_chunk_prefill_noalloc(
+        *[capi.ptr(t) for t in d[:5]], o.data_ptr(), d[5].data_ptr(), sf.data_ptr(), B, T, HV, HK,
+        128, 128, 64, stream) == capi.HIP_SUCCESS
+    assert lib.deltanet_prefill_noalloc_status(stream) == capi.HIP_SUCCESS
+    for i in (slice(0, 1), slice(1, 2), slice(2, 3)):
+        o1, s1 = ops.chunk_prefill(*[t[i] for t in d])
+        assert torch.equal(o[i], o1) and torch.equal(sf[i], s1)
