@@ -428,12 +428,10 @@ def bench_twolevel(ops, dev, reps=10):
         seg_len = max(-(-c // min(segs, c)) if c else 0 for c in nch)
         cus = torch.cuda.get_device_properties(dev).multi_processor_count
 
-        def groups(pairs):
-            # the library's scan instance: 16-column groups while they fit on
-            # the CUs at once, then the paired 32-column and the wide
-            # 64-column instance
-            per = 8 if pairs * 8 <= cus else 4 if pairs * 4 <= cus else 2
-            return -(-pairs // 8) * 8 * per
+        def groups(seqs):
+            # work-groups of the scan instance that the library chooses
+            cols = lib.deltanet_prefill_scan_cols(sum(nch), seqs, HV, HK, cus, 0)
+            return -(-seqs * HV // 8) * 8 * (128 // cols)
 
         nseg = sum(min(segs, c) if c else 1 for c in nch)
         out[name] = {"us_plain": round(ms_plain * 1e3, 2),
@@ -443,8 +441,8 @@ def bench_twolevel(ops, dev, reps=10):
                      "us_replay": round(med[4], 2),
                      "serial_chunks_plain": max(nch),
                      "serial_chunks_twolevel": 2 * seg_len + max(0, min(segs, max(nch)) - 2),
-                     "scan_groups_plain": groups(N * HV),
-                     "scan_groups_per_pass_twolevel": groups(nseg * HV)}
+                     "scan_groups_plain": groups(N),
+                     "scan_groups_per_pass_twolevel": groups(nseg)}
         del ws, d
     return out
 

@@ -20,8 +20,9 @@ extern "C" {
  * time to each kernel).  deltanet_prefill_kernel_count() kernels are launched;
  * events[i] is recorded on `stream` before kernel i and events[count] after
  * the last, so hipEventElapsedTime(events[i], events[i + 1]) is kernel i's
- * duration.  n_events must equal count + 1; the other arguments are as in
- * deltanet_chunk_prefill (dump_debug = 0). */
+ * duration.  The names are the pipeline's (the scan's paired and wide instances
+ * have kernel names of their own).  n_events must equal count + 1; the other
+ * arguments are as in deltanet_chunk_prefill (dump_debug = 0). */
 int deltanet_prefill_kernel_count(void);
 const char* deltanet_prefill_kernel_name(int i);
 hipError_t deltanet_chunk_prefill_timed(const void* q, const void* k, const void* v,
@@ -62,12 +63,11 @@ hipError_t deltanet_chunk_prefill_spin(const void* q, const void* k, const void*
  * with the scan instance chosen by the caller: slice_cols 16 runs one scan
  * work-group per 16 value columns of a (sequence, head), 32 the paired
  * instance with one per 32 columns, 128 the wide instance (the whole head: two
- * work-groups of 64 columns), 0 the library's own choice (16 while its
- * groups fit on the device's CUs at once, then 32, then the wide one; the wide
- * one instead of 32 above 48 heads whose operands come from beyond an L2).  All give
- * bitwise the same o and final state; the wide instance has no bounded waits.  cu_seqlens NULL: num_seqs sequences of
- * T tokens; otherwise a device array [num_seqs + 1] and T the total token
- * count.  spin_limit 0 keeps the library's bounded-wait limit, otherwise as in
+ * work-groups of 64 columns), 0 the library's own choice
+ * (deltanet_prefill_scan_cols).  All give bitwise the same o and final state;
+ * the wide instance has no bounded waits.  cu_seqlens NULL: num_seqs
+ * sequences of T tokens; otherwise a device array [num_seqs + 1] and T the
+ * total token count.  spin_limit 0 keeps the library's bounded-wait limit, otherwise as in
  * deltanet_chunk_prefill_spin.  Other slice_cols: hipErrorInvalidValue. */
 hipError_t deltanet_chunk_prefill_cols(const void* q, const void* k, const void* v,
                                        const float* g, const float* beta, void* o,
@@ -78,8 +78,12 @@ hipError_t deltanet_chunk_prefill_cols(const void* q, const void* k, const void*
 
 /* The scan instance that the library chooses by itself (host only): value
  * columns per work-group, 16, 32 or 64, for `chunks` chunks in all over
- * num_seqs sequences on a device of `cus` CUs, spin_limit as in
- * deltanet_chunk_prefill_cols; -1 for invalid arguments. */
+ * num_seqs sequences on a device of `cus` CUs: 16 while its groups fit on the
+ * CUs at once (heads * 8 <= cus, heads over all sequences), then 32 while its
+ * do (heads * 4 <= cus), then 64; and 64 already above 3/16 cus heads where
+ * HV = HQK or the records exceed 192 MB.  spin_limit as in
+ * deltanet_chunk_prefill_cols; one other than the library's keeps to 16 and
+ * 32.  -1 for invalid arguments. */
 int deltanet_prefill_scan_cols(size_t chunks, int num_seqs, int HV, int HQK, int cus,
                                unsigned spin_limit);
 

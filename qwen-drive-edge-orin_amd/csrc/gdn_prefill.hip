@@ -371,24 +371,25 @@ __device__ bool locate_chunk(const int32_t* cu, int N, int T, int total, int cid
 // scan back ~5 us, with these stores ~1.3 us.  Non-temporal stores (kNt)
 // avoid the write-back too, but the lines then come back from HBM: slower
 // while a call's records fit the 256 MB memory-side cache beside its inputs
-// and o (T1141 HV32 37.2 -> 40.8 us; 100 MB written 3 % slower), faster once
-// they do not, when the scan reads them from HBM either way and the written
-// lines only push older ones out (214 MB written, 2 x 3200 tokens HV32 HK32:
-// 158.0 -> 153.9 us; 209 to 512 MB 3.3-5.5 %; 176 MB the same).  The launcher
-// picks them above kNtRecordBytes written.  The prep never
-// waits for these stores.  The scan's o and state
-// stores stay plain: a wave's later loads complete only after its earlier
-// stores, and waiting behind write-through stores slowed the output waves by
-// more than the write-back they save.  A store of more than 8 bytes reads its data
-// registers after issue: a VALU write to them needs two wait states first,
-// which the compiler inserts after its own stores but cannot see inside an
-// asm statement, so the 16-byte form carries its own s_nop.
+// and o (T1141 HV32 37.2 -> 40.8 us; 80 to 175 MB written 3-12 % slower), faster
+// once they do not, when the scan reads them from HBM either way and the
+// written lines only push older ones out (9000 tokens HV32, 225 MB written:
+// 257 -> 237 us; 8000, 199 MB: 221 -> 213; 7600, 190 MB: 198 -> 203).  The
+// launcher picks them above kNtRecordBytes written.  The prep never waits for
+// these stores.  The state's stores and the 16- and 32-column scans' o stores
+// stay plain: a wave's later loads complete only after its earlier stores, and
+// waiting behind write-through stores slowed the output waves by more than the
+// write-back they save (the wide scan's loaders store o non-temporally, see
+// there).  A store of more than 8 bytes reads its data registers after issue:
+// a VALU write to them needs two wait states first, which the compiler inserts
+// after its own stores but cannot see inside an asm statement, so the 16-byte
+// form carries its own s_nop.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr size_t kNtRecordBytes = size_t(192) << 20;
 // Where records just below that are written through, the prep takes its last
 // chunk first: the scan starts at the first chunks, whose records are then the
 // newest in the memory-side cache (7600 tokens HV32, 190 MB: 198 -> 191 us; 2 x
-// 3600, 182 MB: 152.8 -> 150.1; 172-175 MB within 1 % either way).  With fewer
+// 3600, 182 MB: 152.8 -> 150.1; 172-175 MB within 2 % either way).  With fewer
 // records the first chunk first is the better order (T3200, 80 MB: 84.4 against
 // 85.4; T77 14.38 against 14.45), non-temporally written ones do not care.  The
 // order is an instance of its own: chosen at run time it cost T77 0.05 us.
@@ -2454,8 +2455,8 @@ __global__ __launch_bounds__(kScanThreads, 1) void gdn_scan2_kernel(ScanArgs a) 
 // Bound by the loads where the records come from beyond L2 (75 KB a step at
 // ~36 B/ns per CU: 2.1 us, the same without the compute), by the compute
 // waves' issue and LDS reads where they are in cache (1.6 us, the same without
-// the loads).  8 packed prompts of 19,861 tokens, HV 32: the scan 285 us with
-// the paired instance, 187 with this one; 4 x 1141 tokens 59 and 41.
+// the loads).  8 packed prompts of 19,861 tokens, HV 32: the scan 279 us with
+// the paired instance, 177 with this one; 4 x 1141 tokens 60 and 40.
 // ---------------------------------------------------------------------------
 constexpr int kWideCols = 64;
 constexpr int kWideSlices = kWideCols / kSliceCols;   // 4, one per compute wave
@@ -2546,9 +2547,13 @@ __device__ void run_wide_loader(ScanSmemWide& sm, const ScanArgs& a, const ScanC
         lds_dma16(src, &st.M[j][0]);
         if (j < kTri - kWideLoaders) lds_dma16(src + kWideLoaders * 64, &st.M[j + kWideLoaders][0]);
     };
-    // O of chunk c, rows 16 j .. + 15, whole lines that nothing here reads
-    // again: non-temporal (2 x 3200 tokens HV32 HK32 153.2 -> 148.1 us, 4 x
-    // 1141 HV32 75.0 -> 70.9).  The reads and their wait are one asm
+    // O of chunk c, rows 16 j .. + 15, whole lines that this kernel does not
+    // read again: non-temporal, so that they push no records out of the cache
+    // (plain and non-temporal: 3 x 1141 tokens HV32 67.7 and 66.4 us, 4 x 3200
+    // 206.8 and 204.2, 8 packed prompts 343.7 and 337.1).  A gated RMSNorm
+    // behind the call then finds less of o there: with it, 3 x 300 28.7 and
+    // 28.4, 8 packed prompts 415 and 414, but 4 x 1141 97.4 and 98.7, 2 x 3200
+    // HK32 178.3 and 180.9.  The reads and their wait are one asm
     // block: the compiler would place a wait for every direct-to-LDS load in
     // front of an LDS read of its own.  o's base needs the 8-byte alignment of
     // the narrower instances' stores, no more.
@@ -2892,15 +2897,19 @@ size_t record_bytes(size_t nch, int HV, int HK) {
 // Scan instance (value columns per work-group): 16-column groups while they
 // fit on the CUs at once (one group per CU), the paired 32-column groups once
 // they would run in rounds (then the halves' shared operands halve the
-// rounds), the wide 64-column groups once the paired ones would (paired and
-// wide, 3 x 1141 tokens HV32: 74.7 and 59.8 us; 6 x 256: 43.9 and 35.2; 8
-// packed prompts, 19,861 tokens: 430 and 340), or, with more than 48 heads,
-// where each group's operands come from beyond its L2 (every head has its own
-// Q and K^T, or the records outgrow the memory-side cache) and the wide
-// groups' half as many fetches count (2 x 2000 tokens HV32 HK32: 94.7 and
-// 86.6; 2 x 4096 HV32 HK16: 171 and 166; but 2 x 1141 HV32 HK16 45.5 and 49,
-// and 48 heads 117.5 and 118.7).  A caller's own spin limit keeps to the
-// instances that have bounded waits.
+// rounds), the wide 64-column groups once the paired ones would (calls, paired
+// and wide: 3 x 1141 tokens HV32 92.4 and 67.0 us; 6 x 256 43.8 and 33.8; 9 x 1
+// token HV8 19.0 and 13.1; 8 packed prompts, 19,861 tokens, 430 and 338), or,
+// with more than 48 heads, where every head has its own Q and K^T or the
+// records outgrow the memory-side cache and the wide groups' half as many
+// fetches count.  Its start is shorter too, so 49 to 64 such heads gain at
+// every length (2 x HV32 HK32, paired and wide: 1 token 14.0 and 12.8, 64 14.8
+// and 13.6, 256 20.5 and 19.0, 512 28.1 and 27.6, 1141 62.9 and 58.6, 2000
+// 99.1 and 97.3; 2 x 4096 HV32 HK16 171 and 166; but 48 heads 117.5 and
+// 118.7).  With shared k-heads 64 heads take the paired groups (2 x 1141 HV32
+// HK16 49.9 and 49.6, its scan 32 and 34; up to 256 tokens the wide ones would
+// gain 1.2-1.5 us).  A caller's own spin limit keeps to the instances that
+// have bounded waits.
 int scan_cols(size_t nch, int N, int HV, int HK, long long cus, unsigned spin) {
     const long long heads = (long long)N * HV;
     if (heads * kSlicesPerHead <= cus) return kSliceCols;
